@@ -264,9 +264,13 @@ int launch_dequantize_rows(const DeviceMatrix& m, const std::int32_t* ids, std::
 // done in the GEMV's epilogue with the same two roundings.
 int launch_matmul(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, hipStream_t s,
                   bool accumulate = false);
+// launch_matmul's product for quantized weights and any number of rows, on
+// the matrix cores (qrows.hip); launch_matmul takes it above 8 rows.
+int launch_rows(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, hipStream_t s,
+                bool accumulate);
 // Products of one weight type and input size sharing x and rows (the
-// prefill's q/k/v, gate/up): one split-block launch over all their tiles
-// when each would take the split-block product, else one launch each.
+// prefill's q/k/v, gate/up): one launch over all their tiles when rows > 8
+// and the weights are quantized, else one launch each.
 // RoPE tables (cos_t / sin_t: [position][32], head size 64), the first
 // position of the launch's rows, and one layer's K / V cache ([head][cap][64]).
 struct RopeCache {
@@ -284,9 +288,8 @@ int launch_matmul_shared(const DeviceMatrix* const* ms, const float* const* bias
                          const float* x, std::size_t rows, hipStream_t s, const RopeCache* rope = nullptr,
                          bool* roped = nullptr);
 // The prefill's MLP gate and up projections fused with silu(gate) * up into
-// y, when both would take the split-block product (rows > 8, few tiles, one
-// quantized type and shape); *fused reports whether it ran (else nothing was
-// launched and the caller takes the unfused path).
+// y (rows > 8, one quantized type and shape); *fused reports whether it ran
+// (else nothing was launched and the caller takes the unfused path).
 int launch_gate_up_silu(const DeviceMatrix& gate, const DeviceMatrix& up, const float* x, std::size_t rows,
                         float* y, hipStream_t s, bool* fused);
 // The tolerance-mode one-token step's products (gemv.hip): y += W x' split

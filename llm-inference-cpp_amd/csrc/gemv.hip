@@ -29,13 +29,7 @@
 // (one kernel per row chunk R present); each workgroup runs one tile of one
 // product with the same tile functions.
 //
-// qgemm_exact (batch > 8 on matrices with many tiles, e.g. an lm_head over
-// every position): 64 input rows x 64 outputs per workgroup, 4 x 4 chains
-// per thread, operands from LDS.
-//
-// qgemm_split (batch > 8 on matrices with few tiles, the prefill's
-// projections): a tile's blocks spread over the workgroup's wavefronts,
-// activations from scalar loads, block sums and scales through LDS.
+// Batch > 8 takes the multi-row product (qrows.hip).
 //
 // fp32 weights take kernels::matmul instead (f32.hip).
 #include <algorithm>
@@ -44,86 +38,11 @@
 
 #include "common.hpp"
 #include "glue_math.hpp"
+#include "qblock.hpp"
 
 namespace llmi_hip {
 
 namespace {
-
-// Signed bit-field extract (v_bfe_i32).  The builtin is declared with an
-// unsigned result, so the value is reinterpreted as int before any
-// conversion to float.
-__device__ __forceinline__ int sfield(std::uint32_t w, int offset, int width) {
-  return static_cast<int>(__builtin_amdgcn_sbfe(w, offset, width));
-}
-
-// Global-memory pointers.  The grouped kernel reads its pointers from a
-// table, where the compiler cannot see that they point to global memory;
-// typing them keeps global (not flat) loads for the weights and scalar
-// loads for the activations.
-#define GMEM __attribute__((address_space(1)))
-template <typename T>
-__device__ __forceinline__ const GMEM T* gmem(const T* p) {
-  return (const GMEM T*)p;
-}
-template <typename T>
-__device__ __forceinline__ GMEM T* gmem_out(T* p) {
-  return (GMEM T*)p;
-}
-
-template <int TYPE>
-struct Block {
-  static constexpr int kU = TYPE == LLMI_TYPE_Q8_0 ? 2 : 1;  // 16-byte loads per lane per block
-  uint4 c[kU];
-};
-
-// Weights are streamed through once per product, so the batch 1..8 kernels
-// load them with the nontemporal hint (they are not kept in the caches for
-// reuse); the multi-row prefill kernel re-reads a tile per row chunk and uses
-// ordinary loads.
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-template <bool NT>
-__device__ __forceinline__ uint4 load16(const GMEM uint4* p) {
-  const GMEM u32x4* q = reinterpret_cast<const GMEM u32x4*>(p);
-  const u32x4 v = NT ? __builtin_nontemporal_load(q) : *q;
-  return uint4{v.x, v.y, v.z, v.w};
-}
-template <bool NT>
-__device__ __forceinline__ float loadf(const GMEM float* p) {
-  if (NT) return __builtin_nontemporal_load(p);
-  return *p;
-}
-
-template <int TYPE, bool NT>
-__device__ __forceinline__ Block<TYPE> load_block(const GMEM uint4* __restrict__ codes, std::size_t slot, int lane) {
-  Block<TYPE> b;
-#pragma unroll
-  for (int u = 0; u < Block<TYPE>::kU; ++u) b.c[u] = load16<NT>(codes + (slot * Block<TYPE>::kU + u) * kTileRows + lane);
-  return b;
-}
-
-// The code of element i of a block as float, exactly.
-//   Q4_0: element i is nibble i%8 of word i/8 with +8 bias; XOR-ing every
-//         nibble with 8 turns it into the 4-bit two's complement of n - 8.
-//   Q8_0: element i is signed byte i%4 of word i/4.
-template <int TYPE>
-__device__ __forceinline__ float code_of(const std::uint32_t* w, int i) {
-  if (TYPE == LLMI_TYPE_Q4_0) return static_cast<float>(sfield(w[i >> 3], (i & 7) * 4, 4));
-  return static_cast<float>(sfield(w[i >> 2], (i & 3) * 8, 8));
-}
-
-template <int TYPE>
-__device__ __forceinline__ void unpack_words(const Block<TYPE>& b, std::uint32_t* w) {
-  if (TYPE == LLMI_TYPE_Q4_0) {
-    w[0] = b.c[0].x ^ 0x88888888u;
-    w[1] = b.c[0].y ^ 0x88888888u;
-    w[2] = b.c[0].z ^ 0x88888888u;
-    w[3] = b.c[0].w ^ 0x88888888u;
-  } else {
-    w[0] = b.c[0].x; w[1] = b.c[0].y; w[2] = b.c[0].z; w[3] = b.c[0].w;
-    w[4] = b.c[Block<TYPE>::kU - 1].x; w[5] = b.c[Block<TYPE>::kU - 1].y;
-    w[6] = b.c[Block<TYPE>::kU - 1].z; w[7] = b.c[Block<TYPE>::kU - 1].w;
-  }
-}
 
 // Q4_0 decode constants, kept in VGPRs (v_and_or_b32 takes no literal).
 // Two 4-bit codes n (element value n - 8) are moved into the mantissas of an
@@ -879,436 +798,6 @@ __global__ void __launch_bounds__(64) tsplit_gemv(const uint4* __restrict__ code
   }
 }
 
-// ------------------------------------------------------------ batch > 8
-// The exact multi-row product on many tiles: one workgroup per MR = 64
-// input rows x one 64-row tile of the matrix (64 outputs).  Per quantization
-// block the workgroup stages the block's activations of its MR rows and the
-// block's codes of its 64 outputs, converted to fp32 once, in LDS --
-// transposed, [k][row] and [k][output], so one read gives a thread its 4
-// rows (or 4 outputs) at one k -- plus the 64 scales; double-buffered: the
-// next block's loads go to registers before this block's arithmetic and to
-// LDS after it.  Thread (tr, to) holds the 4 x 4 chains of rows 4tr.. and
-// outputs 4to..4to+3: part = fma(x[k], code[k], part) over the block's k in
-// order, then acc = fma(part, scale, acc) -- the reference's chains, so y is
-// bit-identical.  The final partial block runs only its len elements.
-constexpr int kExactRows = 64;
-
-template <int TYPE>
-__global__ void __launch_bounds__(256) qgemm_exact(const uint4* __restrict__ codes, const float* __restrict__ scales,
-                                                   const float* __restrict__ x, const float* __restrict__ bias,
-                                                   float* __restrict__ y, int in, int nblk, int out, int rows,
-                                                   int accumulate) {
-  constexpr int MR = kExactRows;
-  constexpr int RT = MR / 16;          // rows per thread
-  constexpr int XS = MR + 4;           // LDS floats per k of the activations
-  constexpr int CSTRIDE = kTileRows + 4;
-  constexpr int XPT = MR * kBlock / 256;  // activations staged per thread
-  __shared__ __attribute__((aligned(16))) float xs[2][kBlock * XS];
-  __shared__ __attribute__((aligned(16))) float cs[2][kBlock * CSTRIDE];
-  __shared__ float ss[2][kTileRows];
-  const std::size_t tile = blockIdx.x;
-  const int r0 = blockIdx.y * MR;
-  const int tid = threadIdx.x;
-  const int tr = tid >> 4, to = tid & 15;
-  // Staging: activations of row xr, elements XPT*xq..+XPT-1 of the block;
-  // codes of output cr (= lane of the tile), elements 8*cq..8*cq+7.
-  // Addresses are clamped into x (rows past `rows`, and elements past `in`
-  // of the final block, are never used), so no load sits behind a branch.
-  const int xr = tid / (kBlock / XPT), xq = tid % (kBlock / XPT);
-  const int cr = tid >> 2, cq = tid & 3;
-  const float* xrow = x + static_cast<std::size_t>(min(r0 + xr, rows - 1)) * in;
-  const GMEM uint4* cg = gmem(codes);
-  struct Staged {
-    float xv[XPT];
-    Block<TYPE> blk;
-    float sc;
-  };
-  const auto load = [&](Staged& st, int b) {
-    const int k0 = b * kBlock + XPT * xq;
-#pragma unroll
-    for (int u = 0; u < XPT; ++u) st.xv[u] = xrow[min(k0 + u, in - 1)];
-    st.blk = load_block<TYPE, false>(cg, tile * nblk + b, cr);
-    st.sc = scales[(tile * nblk + b) * kTileRows + (tid & (kTileRows - 1))];
-  };
-  const auto store = [&](const Staged& st, int buf) {
-    std::uint32_t w[8];
-    unpack_words<TYPE>(st.blk, w);
-#pragma unroll
-    for (int u = 0; u < XPT; ++u) xs[buf][(XPT * xq + u) * XS + xr] = st.xv[u];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) cs[buf][(8 * cq + u) * CSTRIDE + cr] = code_of<TYPE>(w, 8 * cq + u);
-    if (tid < kTileRows) ss[buf][tid] = st.sc;
-  };
-  float acc[RT][4];
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-  // Two register sets carry the staged blocks two iterations ahead: set A
-  // the odd blocks, set B the even ones past block 0.  Iteration b computes
-  // block b from LDS, stores block b + 1 (loaded two iterations earlier)
-  // into the other LDS buffer and loads block b + 3 into the set it freed,
-  // so a block's global loads have two blocks of arithmetic to arrive.
-  Staged A, B;
-  load(B, 0);
-  store(B, 0);
-  if (nblk > 1) load(A, 1);
-  if (nblk > 2) load(B, 2);
-  __syncthreads();
-  const auto iteration = [&](int b, Staged& next) {
-    const int buf = b & 1;
-    const int len = min(kBlock, in - b * kBlock);
-    const float* xb = xs[buf] + RT * tr;
-    const float* cb = cs[buf] + 4 * to;
-    float part[RT][4];
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) part[i][j] = 0.0f;
-    const auto step = [&](int k) {
-      const float4 xv = *reinterpret_cast<const float4*>(xb + k * XS);
-      const float xa[RT] = {xv.x, xv.y, xv.z, xv.w};
-      const float4 cv = *reinterpret_cast<const float4*>(cb + k * CSTRIDE);
-      const float ca[4] = {cv.x, cv.y, cv.z, cv.w};
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) part[i][j] = __builtin_fmaf(xa[i], ca[j], part[i][j]);
-    };
-    if (len == kBlock) {
-#pragma unroll 8
-      for (int k = 0; k < kBlock; ++k) step(k);
-    } else {
-      for (int k = 0; k < len; ++k) step(k);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float sc = ss[buf][4 * to + j];
-#pragma unroll
-      for (int i = 0; i < RT; ++i) acc[i][j] = __builtin_fmaf(part[i][j], sc, acc[i][j]);
-    }
-    if (b + 1 < nblk) {
-      store(next, buf ^ 1);
-      if (b + 3 < nblk) load(next, b + 3);
-    }
-    __syncthreads();
-  };
-  for (int b = 0; b < nblk; b += 2) {
-    iteration(b, A);
-    if (b + 1 < nblk) iteration(b + 1, B);
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const std::size_t o = tile * kTileRows + 4 * to + j;
-    if (o >= static_cast<std::size_t>(out)) continue;
-    const float add = bias != nullptr ? bias[o] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < RT; ++i) {
-      const int r = r0 + RT * tr + i;
-      if (r < rows) {
-        float* dst = y + static_cast<std::size_t>(r) * out + o;
-        const float v = acc[i][j] + add;
-        *dst = accumulate ? *dst + v : v;
-      }
-    }
-  }
-}
-
-// qgemm_split (batch > 8, matrices with few 64-row tiles): one workgroup per
-// (tile, chunk of kSplitRows input rows) whose kSplitWaves wavefronts take
-// the tile's blocks round-robin, two per round each (W = kSplitWaves).  In
-// each round wavefront w decodes blocks 2W * round + w and 2W * round + W + w
-// once each (lane l: output tile*64 + l) and forms their block sums for
-// every row of the chunk, with the activations read by scalar loads; the
-// sums and scales go to LDS (two buffers, one barrier per round), and
-// wavefront w then advances the chains of rows w, w + W over the round's 2W
-// blocks in order: acc = fma(part, scale, acc).  (Two blocks per round
-// halve the barriers: Qwen2.5's down_proj at 512 rows 109 -> 102 us.)
-// The block sums are the reference's per-block chains and the chain over
-// blocks runs in block order, so y is bit-identical; splitting the blocks
-// fills the GPU where a 64-row tile per row chunk gives too few workgroups.
-// Small row chunks (2 or 4 rows) measured fastest: the chunk's activations
-// are scalar loads per block and row, and more workgroups hide them.
-template <int TYPE, int kSplitRows, int kSplitWaves, class Epi>
-__device__ __forceinline__ void split_tile(const uint4* __restrict__ codes, const float* __restrict__ scales,
-                                           const float* __restrict__ x, const float* __restrict__ bias, int in,
-                                           int nblk, int out, int rows, std::size_t tile, int chunk, const Epi& epi) {
-  constexpr int RW = (kSplitRows + kSplitWaves - 1) / kSplitWaves;  // chains per lane
-  __shared__ float part[2][kSplitRows][2 * kSplitWaves][kTileRows];
-  __shared__ float scl[2][2 * kSplitWaves][kTileRows];
-  const int r0 = chunk * kSplitRows;
-  const int nr = min(kSplitRows, rows - r0);
-  const int lane = threadIdx.x & (kTileRows - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const GMEM uint4* cg = gmem(codes);
-  const GMEM float* sg = gmem(scales);
-  const GMEM float* xg = gmem(x) + static_cast<std::size_t>(r0) * in;
-  const int nfull = in / kBlock;
-  const std::size_t base = tile * nblk;
-  float acc[RW];
-#pragma unroll
-  for (int i = 0; i < RW; ++i) acc[i] = 0.0f;
-  const int nround = (nblk + 2 * kSplitWaves - 1) / (2 * kSplitWaves);
-  Block<TYPE> cur[2]{};
-  float cur_s[2] = {0.0f, 0.0f};
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int bb = h * kSplitWaves + wave;
-    if (bb < nblk) {
-      cur[h] = load_block<TYPE, false>(cg, base + bb, lane);
-      cur_s[h] = sg[(base + bb) * kTileRows + lane];
-    }
-  }
-  for (int rd = 0; rd < nround; ++rd) {
-    const int buf = rd & 1;
-    Block<TYPE> nxt[2]{};
-    float nxt_s[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int bn = (rd + 1) * 2 * kSplitWaves + h * kSplitWaves + wave;
-      if (bn < nblk) {
-        nxt[h] = load_block<TYPE, false>(cg, base + bn, lane);
-        nxt_s[h] = sg[(base + bn) * kTileRows + lane];
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int b = rd * 2 * kSplitWaves + h * kSplitWaves + wave;
-      const int j = h * kSplitWaves + wave;
-      if (b < nfull) {
-        float c[kBlock];
-        block_codes<TYPE>(cur[h], c);
-#pragma unroll
-        for (int r = 0; r < kSplitRows; ++r)
-          if (r < nr) part[buf][r][j][lane] = codes_dot(c, xg + static_cast<std::size_t>(r) * in + b * kBlock);
-      } else if (b < nblk) {
-        for (int r = 0; r < nr; ++r)
-          part[buf][r][j][lane] =
-              tail_block_dot<TYPE>(cur[h], xg + static_cast<std::size_t>(r) * in + b * kBlock, in - b * kBlock);
-      }
-      if (b < nblk) scl[buf][j][lane] = cur_s[h];
-    }
-    __syncthreads();
-    const int nb = min(2 * kSplitWaves, nblk - rd * 2 * kSplitWaves);
-#pragma unroll
-    for (int i = 0; i < RW; ++i) {
-      const int r = wave + kSplitWaves * i;
-      if (r < kSplitRows && r < nr) {
-        float a = acc[i];
-        for (int j = 0; j < nb; ++j) a = __builtin_fmaf(part[buf][r][j][lane], scl[buf][j][lane], a);
-        acc[i] = a;
-      }
-    }
-    cur[0] = nxt[0];
-    cur[1] = nxt[1];
-    cur_s[0] = nxt_s[0];
-    cur_s[1] = nxt_s[1];
-  }
-  // The epilogue runs on whole wavefronts (row conditions are per wavefront),
-  // so it may exchange values between the lanes of a row.
-  const std::size_t o = tile * kTileRows + lane;
-  const bool o_ok = o < static_cast<std::size_t>(out);
-  const float add = bias != nullptr && o_ok ? bias[o] : 0.0f;
-#pragma unroll
-  for (int i = 0; i < RW; ++i) {
-    const int r = wave + kSplitWaves * i;
-    if (r < kSplitRows && r < nr) epi(r0 + r, o, o_ok, acc[i] + add);
-  }
-}
-
-// y[row][o] = v (or += v).
-struct StoreOut {
-  float* y;
-  int out, accumulate;
-  __device__ __forceinline__ void operator()(int row, std::size_t o, bool o_ok, float v) const {
-    if (!o_ok) return;
-    float* dst = y + static_cast<std::size_t>(row) * out + o;
-    *dst = accumulate ? *dst + v : v;
-  }
-};
-
-template <int TYPE, int R, int W>
-__global__ void __launch_bounds__(W * 64) qgemm_split(const uint4* __restrict__ codes, const float* __restrict__ scales,
-                                                      const float* __restrict__ x, const float* __restrict__ bias,
-                                                      float* __restrict__ y, int in, int nblk, int out, int rows,
-                                                      int accumulate) {
-  split_tile<TYPE, R, W>(codes, scales, x, bias, in, nblk, out, rows, blockIdx.x, blockIdx.y,
-                         StoreOut{y, out, accumulate});
-}
-
-// The gate and up projections of an MLP in one split-block tile: each round
-// a wavefront decodes block b of the gate matrix and forms its block sums for
-// every input row, then the same for the up matrix, the chains run side by
-// side, and the epilogue writes
-// silu(gate) * up as the reference's MLP does after its two matmuls
-// (kernels.cpp:148, transformer.cpp:288-290): v = gate + 0.0f (the matmul's
-// absent bias), v / (1 + expf(-v)) * (up + 0.0f), with the exact expf.
-template <int TYPE, int kSplitRows, int kSplitWaves>
-__global__ void __launch_bounds__(kSplitWaves * 64) qgemm_split_gate_up(
-    const uint4* __restrict__ codes_g, const float* __restrict__ scales_g, const uint4* __restrict__ codes_u,
-    const float* __restrict__ scales_u, const float* __restrict__ x, float* __restrict__ y, int in, int nblk, int out,
-    int rows) {
-  constexpr int RW = (kSplitRows + kSplitWaves - 1) / kSplitWaves;  // chains per lane and product
-  __shared__ float part[2][2][kSplitRows][kSplitWaves][kTileRows];  // [buffer][gate, up]
-  __shared__ float scl[2][2][kSplitWaves][kTileRows];
-  const std::size_t tile = blockIdx.x;
-  const int r0 = blockIdx.y * kSplitRows;
-  const int nr = min(kSplitRows, rows - r0);
-  const int lane = threadIdx.x & (kTileRows - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const GMEM uint4* cgg = gmem(codes_g);
-  const GMEM uint4* cgu = gmem(codes_u);
-  const GMEM float* sgg = gmem(scales_g);
-  const GMEM float* sgu = gmem(scales_u);
-  const GMEM float* xg = gmem(x) + static_cast<std::size_t>(r0) * in;
-  const int nfull = in / kBlock;
-  const std::size_t base = tile * nblk;
-  float acc_g[RW], acc_u[RW];
-#pragma unroll
-  for (int i = 0; i < RW; ++i) acc_g[i] = acc_u[i] = 0.0f;
-  const int nround = (nblk + kSplitWaves - 1) / kSplitWaves;
-  Block<TYPE> cur_g{}, cur_u{};
-  float sc_g = 0.0f, sc_u = 0.0f;
-  if (wave < nblk) {
-    cur_g = load_block<TYPE, false>(cgg, base + wave, lane);
-    cur_u = load_block<TYPE, false>(cgu, base + wave, lane);
-    sc_g = sgg[(base + wave) * kTileRows + lane];
-    sc_u = sgu[(base + wave) * kTileRows + lane];
-  }
-  for (int rd = 0; rd < nround; ++rd) {
-    const int buf = rd & 1;
-    const int b = rd * kSplitWaves + wave;
-    Block<TYPE> nxt_g{}, nxt_u{};
-    float nsc_g = 0.0f, nsc_u = 0.0f;
-    if (b + kSplitWaves < nblk) {
-      nxt_g = load_block<TYPE, false>(cgg, base + b + kSplitWaves, lane);
-      nxt_u = load_block<TYPE, false>(cgu, base + b + kSplitWaves, lane);
-      nsc_g = sgg[(base + b + kSplitWaves) * kTileRows + lane];
-      nsc_u = sgu[(base + b + kSplitWaves) * kTileRows + lane];
-    }
-    if (b < nfull) {
-      // One product's block at a time: a single set of 32 decoded codes
-      // stays live, which keeps the kernel at the split kernel's occupancy.
-      {
-        float c[kBlock];
-        block_codes<TYPE>(cur_g, c);
-#pragma unroll
-        for (int r = 0; r < kSplitRows; ++r)
-          if (r < nr) part[buf][0][r][wave][lane] = codes_dot(c, xg + static_cast<std::size_t>(r) * in + b * kBlock);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      {
-        float c[kBlock];
-        block_codes<TYPE>(cur_u, c);
-#pragma unroll
-        for (int r = 0; r < kSplitRows; ++r)
-          if (r < nr) part[buf][1][r][wave][lane] = codes_dot(c, xg + static_cast<std::size_t>(r) * in + b * kBlock);
-      }
-    } else if (b < nblk) {
-      for (int r = 0; r < nr; ++r) {
-        const GMEM float* xr = xg + static_cast<std::size_t>(r) * in + b * kBlock;
-        part[buf][0][r][wave][lane] = tail_block_dot<TYPE>(cur_g, xr, in - b * kBlock);
-        part[buf][1][r][wave][lane] = tail_block_dot<TYPE>(cur_u, xr, in - b * kBlock);
-      }
-    }
-    if (b < nblk) {
-      scl[buf][0][wave][lane] = sc_g;
-      scl[buf][1][wave][lane] = sc_u;
-    }
-    __syncthreads();
-    const int nb = min(kSplitWaves, nblk - rd * kSplitWaves);
-#pragma unroll
-    for (int i = 0; i < RW; ++i) {
-      const int r = wave + kSplitWaves * i;
-      if (r < kSplitRows && r < nr) {
-        float ag = acc_g[i], au = acc_u[i];
-        for (int j = 0; j < nb; ++j) {
-          ag = __builtin_fmaf(part[buf][0][r][j][lane], scl[buf][0][j][lane], ag);
-          au = __builtin_fmaf(part[buf][1][r][j][lane], scl[buf][1][j][lane], au);
-        }
-        acc_g[i] = ag;
-        acc_u[i] = au;
-      }
-    }
-    cur_g = nxt_g;
-    cur_u = nxt_u;
-    sc_g = nsc_g;
-    sc_u = nsc_u;
-  }
-  const std::size_t o = tile * kTileRows + lane;
-  if (o < static_cast<std::size_t>(out)) {
-#pragma unroll
-    for (int i = 0; i < RW; ++i) {
-      const int r = wave + kSplitWaves * i;
-      if (r < kSplitRows && r < nr) {
-        const float v = acc_g[i] + 0.0f;
-        const float u = acc_u[i] + 0.0f;
-        y[static_cast<std::size_t>(r0 + r) * out + o] = v / (1.0f + exact::expf(-v)) * u;
-      }
-    }
-  }
-}
-
-// Up to kMaxShared products of one weight type and input size that share x
-// and rows (the prefill's q/k/v, gate/up) in one launch: workgroup column
-// blockIdx.x is tile blockIdx.x - tile_end[p - 1] of the product p whose
-// tile range holds it.
-constexpr int kMaxShared = 3;
-struct SplitGroup {
-  const uint4* codes[kMaxShared];
-  const float* scales[kMaxShared];
-  const float* bias[kMaxShared];
-  float* y[kMaxShared];
-  int out[kMaxShared];
-  int tile_end[kMaxShared];
-  int mode[kMaxShared];  // a SharedEpilogue
-  int count;
-  RopeCache rope;
-};
-
-// A product's output in a grouped launch: y as computed, RoPE'd in place (q),
-// RoPE'd into the KV cache (k), or copied into it (v).  The RoPE modes take a
-// head size of 64, one head per 64-output tile, and rotate elements (i, i+32)
-// of a head with the host tables: v[i] = fma(a, c, -(b * s)),
-// v[i + 32] = fma(b, c, a * s) (kernels.cpp:122-134).
-struct GroupStore {
-  const SplitGroup& g;
-  int p;
-  __device__ __forceinline__ void operator()(int row, std::size_t o, bool o_ok, float v) const {
-    const int mode = g.mode[p];
-    if (mode == kStorePlain) {
-      if (o_ok) g.y[p][static_cast<std::size_t>(row) * g.out[p] + o] = v;
-      return;
-    }
-    const int lane = static_cast<int>(o & 63);
-    const int pos = g.rope.base + row;
-    if (mode != kStoreCache) {
-      const float partner = __shfl_xor(v, 32, 64);
-      const float c = g.rope.cos_t[static_cast<std::size_t>(pos) * 32 + (lane & 31)];
-      const float sn = g.rope.sin_t[static_cast<std::size_t>(pos) * 32 + (lane & 31)];
-      v = lane < 32 ? __builtin_fmaf(v, c, -(partner * sn)) : __builtin_fmaf(v, c, partner * sn);
-    }
-    if (!o_ok) return;
-    if (mode == kStoreRope) {
-      g.y[p][static_cast<std::size_t>(row) * g.out[p] + o] = v;
-    } else {
-      const std::size_t head = o >> 6;
-      g.y[p][(head * g.rope.cap + pos) * 64 + lane] = v;
-    }
-  }
-};
-
-template <int TYPE, int R, int W>
-__global__ void __launch_bounds__(W * 64) qgemm_split_group(SplitGroup g, const float* __restrict__ x, int in,
-                                                            int nblk, int rows) {
-  const int t = static_cast<int>(blockIdx.x);
-  int p = 0;
-  while (p + 1 < g.count && t >= g.tile_end[p]) ++p;
-  const int t0 = p == 0 ? 0 : g.tile_end[p - 1];
-  split_tile<TYPE, R, W>(g.codes[p], g.scales[p], x, g.bias[p], in, nblk, g.out[p], rows,
-                         static_cast<std::size_t>(t - t0), blockIdx.y, GroupStore{g, p});
-}
-
 // ------------------------------------------------------------ planning
 // LDS bytes of one workgroup of each kind.
 // part[nr][nblk][64], scale[nblk][64], then the chain's look-ahead padding.
@@ -1353,7 +842,7 @@ int narrow_waves(std::size_t nblk) {
 }
 
 struct TilePlan {
-  int kind = 0;  // 0: qgemm_exact; GroupProblem::kNarrow; or the row chunk R of qgemv_tile
+  int kind = 0;  // 0: the multi-row product (qrows.hip); GroupProblem::kNarrow; or the row chunk R of qgemv_tile
   int waves = 1;
   int bpw = 1;
   std::size_t lds = 0;
@@ -1366,7 +855,7 @@ TilePlan plan_single(const DeviceMatrix& m, std::size_t rows) {
   constexpr std::size_t kNarrowTiles = 128;
   const std::size_t nblk = std::max<std::size_t>(m.nblk, 1);
   TilePlan p;
-  if (rows > 8) return p;  // qgemm_exact
+  if (rows > 8) return p;
   if (rows == 1 && m.ntiles < kNarrowTiles && narrow_lds(m.in, nblk) <= max_lds_per_block()) {
     p.kind = GroupProblem::kNarrow;
     p.waves = narrow_waves(nblk);
@@ -1376,7 +865,7 @@ TilePlan plan_single(const DeviceMatrix& m, std::size_t rows) {
   }
   int r = pick_chunk(rows, nblk, kLdsTarget);
   if (r == 0) r = pick_chunk(1, nblk, max_lds_per_block());
-  if (r == 0) return p;  // rows too long for LDS staging: qgemm_exact
+  if (r == 0) return p;  // rows too long for LDS staging
   p.kind = r;
   p.bpw = static_cast<int>(ceil_div(nblk, wide_waves(nblk, m.type)));
   p.waves = static_cast<int>(ceil_div(nblk, p.bpw));
@@ -1393,66 +882,10 @@ void launch_tile(const DeviceMatrix& m, const float* x, std::size_t rows, const 
       static_cast<int>(m.out), static_cast<int>(rows), p.bpw, acc);
 }
 
-template <int TYPE, int R, int W>
-void launch_split(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, int acc,
-                  hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(m.ntiles), static_cast<unsigned>(ceil_div(rows, R)));
-  qgemm_split<TYPE, R, W><<<grid, W * 64, 0, s>>>(reinterpret_cast<const uint4*>(m.codes), m.scales, x, bias, y,
-                                                  static_cast<int>(m.in), static_cast<int>(m.nblk),
-                                                  static_cast<int>(m.out), static_cast<int>(rows), acc);
-}
-
-// Multi-row products.  qgemm_exact when its 64-row chunks alone give about
-// 1024 workgroups (an lm_head over every position); otherwise qgemm_split
-// with the row chunk and wavefront count measured fastest on MI355X for the
-// launch's size: 4 rows x 4 wavefronts from ~6K wavefronts up, 4 x 8 from
-// ~4K, else 2 x 8 (SmolLM2-135M and Qwen2.5-0.5B projections at 128 and 512
-// rows; Qwen2.5's gate/up 92 us split against 109 on qgemm_exact, its
-// 151936-row lm_head 2.46 ms split against 2.14).
-template <int TYPE>
-void launch_rows(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, int acc,
-                 hipStream_t s) {
-  constexpr std::size_t kExactMin = 1024;
-  if (m.ntiles * ceil_div(rows, kExactRows) >= kExactMin) {
-    const dim3 grid(static_cast<unsigned>(m.ntiles), static_cast<unsigned>(ceil_div(rows, kExactRows)));
-    qgemm_exact<TYPE><<<grid, 256, 0, s>>>(reinterpret_cast<const uint4*>(m.codes), m.scales, x, bias, y,
-                                           static_cast<int>(m.in), static_cast<int>(m.nblk), static_cast<int>(m.out),
-                                           static_cast<int>(rows), acc);
-    return;
-  }
-  // Here ntiles * ceil(rows / 64) < 1024, so rows < 65536 and every split
-  // launch's grid y (ceil(rows / R), R >= 2) stays below 32768.
-  const auto waves = [&](std::size_t r, std::size_t w) { return m.ntiles * ceil_div(rows, r) * w; };
-  if (waves(4, 4) >= 6144) launch_split<TYPE, 4, 4>(m, x, rows, bias, y, acc, s);
-  else if (waves(4, 8) >= 4096) launch_split<TYPE, 4, 8>(m, x, rows, bias, y, acc, s);
-  else launch_split<TYPE, 2, 8>(m, x, rows, bias, y, acc, s);
-}
-
-template <int TYPE, int R, int W>
-void launch_split_group(const SplitGroup& g, std::size_t tiles, const float* x, std::size_t in, std::size_t nblk,
-                        std::size_t rows, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(ceil_div(rows, R)));
-  qgemm_split_group<TYPE, R, W><<<grid, W * 64, 0, s>>>(g, x, static_cast<int>(in), static_cast<int>(nblk),
-                                                        static_cast<int>(rows));
-}
-
-// The grouped split launch of launch_matmul_shared: the row chunk and
-// wavefront count by the launch's total size, as for one product.
-template <int TYPE>
-void launch_group_rows(const SplitGroup& g, std::size_t tiles, const float* x, std::size_t in, std::size_t nblk,
-                       std::size_t rows, hipStream_t s) {
-  const auto waves = [&](std::size_t r, std::size_t w) { return tiles * ceil_div(rows, r) * w; };
-  if (waves(4, 4) >= 6144) launch_split_group<TYPE, 4, 4>(g, tiles, x, in, nblk, rows, s);
-  else if (waves(4, 8) >= 4096) launch_split_group<TYPE, 4, 8>(g, tiles, x, in, nblk, rows, s);
-  else launch_split_group<TYPE, 2, 8>(g, tiles, x, in, nblk, rows, s);
-}
-
 template <int TYPE>
 void launch_typed(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, int acc,
-                  hipStream_t s) {
-  const TilePlan p = plan_single(m, rows);
+                  const TilePlan& p, hipStream_t s) {
   switch (p.kind) {
-    case 0: launch_rows<TYPE>(m, x, rows, bias, y, acc, s); break;
     case GroupProblem::kNarrow:
       qgemv_narrow<TYPE><<<static_cast<unsigned>(ceil_div(m.out, 16)), static_cast<unsigned>(p.waves * 64), p.lds, s>>>(
           reinterpret_cast<const uint4*>(m.codes), m.scales, x, bias, y, static_cast<int>(m.in),
@@ -1483,95 +916,11 @@ int launch_matmul(const DeviceMatrix& m, const float* x, std::size_t rows, const
   }
   if (int rc = check_shape(m, rows)) return rc;
   LLMI_REQUIRE(x != nullptr && y != nullptr, "matmul: null pointer");
+  const TilePlan p = plan_single(m, rows);
+  if (p.kind == 0) return launch_rows(m, x, rows, bias, y, s, accumulate);
   const int acc = accumulate ? 1 : 0;
-  if (m.type == LLMI_TYPE_Q8_0) launch_typed<LLMI_TYPE_Q8_0>(m, x, rows, bias, y, acc, s);
-  else launch_typed<LLMI_TYPE_Q4_0>(m, x, rows, bias, y, acc, s);
-  LLMI_TRY_HIP(hipGetLastError());
-  return LLMI_OK;
-}
-
-int launch_gate_up_silu(const DeviceMatrix& gate, const DeviceMatrix& up, const float* x, std::size_t rows,
-                        float* y, hipStream_t s, bool* fused) {
-  *fused = false;
-  if (rows <= 8 || gate.type == LLMI_TYPE_F32 || gate.type != up.type || gate.in != up.in || gate.out != up.out ||
-      gate.out == 0 || gate.ntiles * ceil_div(rows, kExactRows) >= 1024)
-    return LLMI_OK;
-  if (int rc = check_shape(gate, rows)) return rc;
-  LLMI_REQUIRE(x != nullptr && y != nullptr, "gate_up: null pointer");
-  const auto waves = [&](std::size_t r, std::size_t w) { return gate.ntiles * ceil_div(rows, r) * w; };
-  const auto launch = [&](auto tag_r, auto tag_w) {
-    constexpr int R = decltype(tag_r)::value, W = decltype(tag_w)::value;
-    const dim3 grid(static_cast<unsigned>(gate.ntiles), static_cast<unsigned>(ceil_div(rows, R)));
-    const int in = static_cast<int>(gate.in), nblk = static_cast<int>(gate.nblk), out = static_cast<int>(gate.out);
-    const int nr = static_cast<int>(rows);
-    const auto* cg = reinterpret_cast<const uint4*>(gate.codes);
-    const auto* cu = reinterpret_cast<const uint4*>(up.codes);
-    if (gate.type == LLMI_TYPE_Q8_0)
-      qgemm_split_gate_up<LLMI_TYPE_Q8_0, R, W><<<grid, W * 64, 0, s>>>(cg, gate.scales, cu, up.scales, x, y, in, nblk,
-                                                                        out, nr);
-    else
-      qgemm_split_gate_up<LLMI_TYPE_Q4_0, R, W><<<grid, W * 64, 0, s>>>(cg, gate.scales, cu, up.scales, x, y, in, nblk,
-                                                                        out, nr);
-  };
-  using I2 = std::integral_constant<int, 2>;
-  using I4 = std::integral_constant<int, 4>;
-  using I8 = std::integral_constant<int, 8>;
-  if (waves(4, 4) >= 6144) launch(I4{}, I4{});
-  else if (waves(4, 8) >= 4096) launch(I4{}, I8{});
-  else launch(I2{}, I8{});
-  LLMI_TRY_HIP(hipGetLastError());
-  *fused = true;
-  return LLMI_OK;
-}
-
-int launch_matmul_shared(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys, int count,
-                         const float* x, std::size_t rows, hipStream_t s, const RopeCache* rope, bool* roped) {
-  if (roped != nullptr) *roped = false;
-  LLMI_REQUIRE(count >= 1 && count <= kMaxShared, "matmul_shared: 1..3 products");
-  std::size_t tiles = 0;
-  bool grouped = count > 1 && rows > 8;
-  for (int i = 0; i < count && grouped; ++i) {
-    const DeviceMatrix& m = *ms[i];
-    // One launch only where each product alone would take qgemm_split.
-    grouped = m.type != LLMI_TYPE_F32 && m.type == ms[0]->type && m.in == ms[0]->in && m.out > 0 &&
-              m.ntiles * ceil_div(rows, kExactRows) < 1024;
-    tiles += m.ntiles;
-  }
-  if (!grouped) {
-    for (int i = 0; i < count; ++i)
-      if (int rc = launch_matmul(*ms[i], x, rows, biases[i], ys[i], s)) return rc;
-    return LLMI_OK;
-  }
-  if (int rc = check_shape(*ms[0], rows)) return rc;
-  LLMI_REQUIRE(x != nullptr, "matmul_shared: null x");
-  SplitGroup g{};
-  int end = 0;
-  for (int i = 0; i < count; ++i) {
-    LLMI_REQUIRE(ys[i] != nullptr, "matmul_shared: null y");
-    g.codes[i] = reinterpret_cast<const uint4*>(ms[i]->codes);
-    g.scales[i] = ms[i]->scales;
-    g.bias[i] = biases[i];
-    g.y[i] = ys[i];
-    g.out[i] = static_cast<int>(ms[i]->out);
-    end += static_cast<int>(ms[i]->ntiles);
-    g.tile_end[i] = end;
-    g.mode[i] = kStorePlain;
-  }
-  g.count = count;
-  // RoPE and the cache writes ride along for q, k, v of head size 64.
-  if (rope != nullptr && roped != nullptr && count == 3 && ms[0]->out % 64 == 0 && ms[1]->out % 64 == 0 &&
-      ms[2]->out % 64 == 0) {
-    g.rope = *rope;
-    g.mode[0] = kStoreRope;
-    g.mode[1] = kStoreRopeCache;
-    g.mode[2] = kStoreCache;
-    g.y[1] = rope->kc;
-    g.y[2] = rope->vc;
-    *roped = true;
-  }
-  const DeviceMatrix& m0 = *ms[0];
-  if (m0.type == LLMI_TYPE_Q8_0) launch_group_rows<LLMI_TYPE_Q8_0>(g, tiles, x, m0.in, m0.nblk, rows, s);
-  else launch_group_rows<LLMI_TYPE_Q4_0>(g, tiles, x, m0.in, m0.nblk, rows, s);
+  if (m.type == LLMI_TYPE_Q8_0) launch_typed<LLMI_TYPE_Q8_0>(m, x, rows, bias, y, acc, p, s);
+  else launch_typed<LLMI_TYPE_Q4_0>(m, x, rows, bias, y, acc, p, s);
   LLMI_TRY_HIP(hipGetLastError());
   return LLMI_OK;
 }

@@ -1,0 +1,73 @@
+"""The exact multi-row product (csrc/qrows.hip, more than 8 input rows)
+against the oracle, bit for bit, on the shapes where its tiles and its
+dispatch can go wrong."""
+
+import numpy as np
+import pytest
+
+import llmi_hip as H
+import oracle as O
+import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
+
+
+# (rows, out, in): one side and the other of a 16- and 32-row tile, of a
+# 16-output group and a 64-row tile, of a partial block and a whole one, of
+# one block per wavefront (4, 8, 16 wavefronts) and several; 16 x 16 tiles up
+# to 256 (16 wavefronts a tile), up to 1408 / 2560 (8), up to 8191 (16 rows a
+# wavefront) and from 8192 (32 rows).
+SHAPES = [(9, 1, 1), (16, 15, 31), (17, 16, 32), (31, 17, 33), (32, 63, 63), (33, 65, 512), (15, 64, 513),
+          (40, 130, 1055), (100, 700, 260), (48, 1500, 1024), (257, 1416, 64), (260, 1500, 1037), (529, 3900, 96),
+          (545, 3890, 35)]
+
+
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("rows,out,n_in", SHAPES)
+def test_tile_edges_match_oracle(qt, rows, out, n_in):
+    """Also with x only 4-byte aligned, and next to values that must not be
+    read as its padding."""
+    orc = O.oracle()
+    w = synth.normal(out * 5 + n_in, out * n_in, 0.0, 0.02)
+    x = synth.normal(rows * 11 + n_in, rows * n_in, 0.0, 1.0)
+    bias = synth.normal(3, out, 0.0, 0.5)
+    data, scales = orc.quantize(w, out, n_in, qt)
+    dev = H.Weight.upload(data, scales, out, n_in, qt)
+    want = orc.matmul(x, rows, n_in, data, scales, qt, out, bias)
+    around = np.full(rows * n_in + 9, np.nan, dtype=np.float32)
+    around[1 : 1 + rows * n_in] = x
+    xd, bd = H.DeviceBuffer.from_array(around), H.DeviceBuffer.from_array(bias)
+    yd = H.DeviceBuffer.from_array(np.full(rows * out + 64, 7.0, dtype=np.float32))
+    dev.matmul_dev(xd.ptr + 4, rows, bd.ptr, yd.ptr)
+    H.synchronize()
+    got = yd.download(np.float32)
+    assert np.array_equal(bits(got[: rows * out]), bits(want))
+    assert np.all(got[rows * out :] == 7.0)
+
+
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+def test_extreme_rows_stay_in_their_rows(qt):
+    """Subnormal, zero, huge and infinite activations: each row's results are
+    the oracle's, whatever its neighbours in the tile hold."""
+    orc = O.oracle()
+    rows, out, n_in = 24, 80, 96
+    w = synth.normal(1, out * n_in, 0.0, 0.02)
+    x = synth.normal(2, rows * n_in, 0.0, 1.0).reshape(rows, n_in)
+    x[1] *= np.float32(1e-42)
+    x[2] = 0.0
+    x[3] = -0.0
+    x[4] *= np.float32(1e36)
+    x[5, 7] = np.inf
+    x[6] *= np.float32(1e-30)
+    data, scales = orc.quantize(w, out, n_in, qt)
+    scales[::7] *= np.float32(1e-12)
+    dev = H.Weight.upload(data, scales, out, n_in, qt)
+    got = dev.matmul(x.reshape(-1), rows, None)
+    want = orc.matmul(x.reshape(-1), rows, n_in, data, scales, qt, out, None)
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(bits(got)[~nan], bits(want)[~nan])
