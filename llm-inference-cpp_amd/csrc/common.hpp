@@ -94,7 +94,9 @@ __host__ __device__ inline int attn_chunk_len(int npos) {
 
 // One product of a grouped launch (qgemv_group), as the kernel reads it.
 struct GroupProblem {
-  static constexpr int kNarrow = 16;  // kind: 16-row tiles, batch 1; else the row chunk R (1, 2, 4, 8)
+  // kind: 16-row tiles, batch 1; 64-row tiles with up to 4 or 8 input rows on
+  // the matrix cores; else 64-row tiles on the vector ALUs, row chunk 1, 2, 4.
+  static constexpr int kNarrow = 16, kFew4 = 104, kFew8 = 108;
   const std::uint8_t* codes;
   const float* scales;
   const float* x;
@@ -118,8 +120,8 @@ struct GroupEntry {
   const float* pw = nullptr;
   float eps = 0.0f;
 };
-// One kernel launch of a group: the products of weight type `type` and row
-// chunk `rchunk` (GroupProblem::kNarrow: the 16-row tiles), at
+// One kernel launch of a group: the products of weight type `type` and kind
+// `rchunk` (as GroupProblem::kind), at
 // probs[prob_offset...], workgroup w running product wg_prob[map_offset + w].
 struct GroupLaunch {
   int type = 0, rchunk = 1, waves = 1, total_wgs = 0, nprob = 0;

@@ -14,22 +14,26 @@
 // broadcast to the fused multiply-adds.  Every code byte and scale is read
 // from HBM once; the kernels are HBM-bound at batch 1.
 //
-// qgemv_tile (batch 1..8): one workgroup per (64-row tile, chunk of up to R
-// input rows).  Its W wavefronts split the tile's blocks into contiguous
-// ranges; each decodes a block once and forms the block sums of every input
-// row of the chunk, which it parks in LDS together with the block scales.
-// After one barrier the wavefronts run the sequential chains over all blocks
-// (one chain per input row), add the bias and store y.  Splitting the blocks
-// over wavefronts is what fills the GPU when a matrix has few tiles.
+// qgemv_tile (batch 1; 2 and 3 rows and long rows by few_kind): one workgroup
+// per (64-row tile, chunk of up to R input rows).  Its W wavefronts split the
+// tile's blocks into contiguous ranges; each decodes a block once and forms
+// the block sums of every input row of the chunk, which it parks in LDS
+// together with the block scales.  After one barrier the wavefronts run the
+// sequential chains over all blocks (one chain per input row), add the bias
+// and store y.  Splitting the blocks over wavefronts is what fills the GPU
+// when a matrix has few tiles.
+//
+// qgemv_few (2..8 rows): a 64-row tile on the matrix cores (qfew.hpp).
 //
 // qgemv_narrow (batch 1, matrices with few rows): 16-row tiles, 4x the
 // workgroups of qgemv_tile.
 //
-// qgemv_group: a fixed list of products (each batch 1..8) launched together
-// (one kernel per row chunk R present); each workgroup runs one tile of one
-// product with the same tile functions.
+// qgemv_group, qgemv_group_few: a fixed list of products (each batch 1..8)
+// launched together (one kernel per kind of tile present); each workgroup
+// runs one tile of one product with the same tile functions.
 //
-// Batch > 8 takes the multi-row product (qrows.hip).
+// Batch > 8, and few rows on few tiles, take the multi-row product
+// (qrows.hip).
 //
 // fp32 weights take kernels::matmul instead (f32.hip).
 #include <algorithm>
@@ -39,6 +43,7 @@
 #include "common.hpp"
 #include "glue_math.hpp"
 #include "qblock.hpp"
+#include "qfew.hpp"
 
 namespace llmi_hip {
 
@@ -519,6 +524,16 @@ __global__ void __launch_bounds__(1024) qgemv_tile(const uint4* __restrict__ cod
                      lds);
 }
 
+// Up to R = 4 or 8 input rows on the matrix cores (qfew.hpp): one workgroup of W wavefronts per 64-row tile.
+template <int TYPE, int R, int W>
+__global__ void __launch_bounds__(64 * W, 2) qgemv_few(const uint4* __restrict__ codes, const float* __restrict__ scales,
+                                                    const float* __restrict__ x, int in, int nblk, int rows, int out,
+                                                    const float* __restrict__ bias, float* __restrict__ y,
+                                                    int accumulate) {
+  few::tile<TYPE, R, W>(gmem(codes), gmem(scales), gmem(x), gmem(bias), gmem_out(y), in, nblk, out, rows, accumulate,
+                        blockIdx.x);
+}
+
 template <int TYPE>
 __global__ void __launch_bounds__(1024) qgemv_narrow(const uint4* __restrict__ codes, const float* __restrict__ scales,
                                                      const float* __restrict__ x, const float* __restrict__ bias,
@@ -550,6 +565,17 @@ __global__ void __launch_bounds__(1024) qgemv_group(const GroupProblem* __restri
   const GMEM float* x = gmem(p.x + static_cast<std::size_t>(r0) * p.in);
   GMEM float* y = gmem_out(p.y + static_cast<std::size_t>(r0) * p.out);
   wide_tile<TYPE, R>(codes, scales, x, bias, y, p.in, p.nblk, p.out, nr, p.bpw, p.accumulate, tile, lds);
+}
+
+// The same for products on the matrix cores (kinds kFew4 and kFew8).
+template <int TYPE, int R, int W>
+__global__ void __launch_bounds__(64 * W, 2) qgemv_group_few(const GroupProblem* __restrict__ probs,
+                                                          const std::uint32_t* __restrict__ wg_prob) {
+  const int wg = blockIdx.x;
+  const int idx = __builtin_amdgcn_readfirstlane(static_cast<int>(wg_prob[wg]));
+  const GroupProblem p = probs[idx];
+  few::tile<TYPE, R, W>(gmem(reinterpret_cast<const uint4*>(p.codes)), gmem(p.scales), gmem(p.x), gmem(p.bias),
+                        gmem_out(p.y), p.in, p.nblk, p.out, p.rows, p.accumulate, wg - p.first_wg);
 }
 
 // The 16-row tiles of a group (batch 1, optional prologue), in a kernel of
@@ -815,15 +841,40 @@ std::size_t narrow_lds(std::size_t in, std::size_t nblk) {
 // a CU; longer rows may use up to the per-workgroup maximum.
 constexpr std::size_t kLdsTarget = 64 * 1024;
 
-// Row chunk R (a template size: 1, 2, 4, 8) of a wide workgroup: the
-// smallest one covering `rows`, halved until its LDS fits `budget`; 0 if not
-// even one row fits.
-int pick_chunk(std::size_t rows, std::size_t nblk, std::size_t budget) {
-  const int want = rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8;
-  for (int r = want; r >= 1; r /= 2)
-    if (wide_lds(nblk, std::min<std::size_t>(rows, r)) <= budget) return r;
-  return 0;
+// Whether a 64-row tile's block sums of one input row fit LDS (in up to ~10k).
+bool wide_fits(std::size_t nblk) { return wide_lds(nblk, 1) <= max_lds_per_block(); }
+
+// Row chunk R (1, 2 or 4) of a wide workgroup on the vector ALUs, at most
+// `want`, halved until its LDS fits.
+int pick_chunk(int want, std::size_t rows, std::size_t nblk) {
+  for (int r = want; r > 1; r /= 2)
+    if (wide_lds(nblk, std::min<std::size_t>(rows, r)) <= kLdsTarget) return r;
+  return 1;
 }
+
+// How a launch of `tiles` 64-row tiles runs a product of 2..8 rows on 64-row
+// tiles (GroupProblem's kinds), by measurement (us, vector ALUs / matrix
+// cores, Q4_0 and Q8_0):
+//   2 rows: the vector ALUs -- half of a 4-row matrix instruction's rows are
+//     empty -- (151936 x 896 20.4 / 24.6, 4864 x 896 4.6 / 5.0) except for
+//     Q8_0, whose codes decode for less, on many tiles (32.6 / 25.7), and for a
+//     partial last block (30000 x 700 8.0 / 5.9);
+//   3 rows of Q4_0 on many tiles: 49152 x 576 6.7 / 7.4;
+//   rows of more than 64 blocks on few tiles: row chunks on several
+//     workgroups (896 x 4864 10.4 / 15.2);
+//   else the matrix cores (151936 x 896 at 8 rows 52.3 / 33.6 and 78.2 /
+//     35.6, at 4 27.9 / 24.2 and 41.7 / 26.3).
+int few_kind(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
+  if (m.nblk > 64 && tiles < 128) return pick_chunk(4, rows, m.nblk);
+  if (rows == 2 && m.in % kBlock == 0 && (m.type == LLMI_TYPE_Q4_0 || tiles < 512)) return pick_chunk(2, rows, m.nblk);
+  if (rows == 3 && m.type == LLMI_TYPE_Q4_0 && tiles >= 512 && pick_chunk(4, rows, m.nblk) == 4) return 4;
+  return rows <= 4 ? GroupProblem::kFew4 : GroupProblem::kFew8;
+}
+
+// Wavefronts per tile on the matrix cores (4, 8 or 16; us at 8 rows, Q4_0): by
+// the tiles, enough to fill the GPU (768 tiles of 576 inputs 9.3 / 10.2 /
+// 12.5; 256 of 896 7.5 / 6.8 / 7.3; 76 7.2 / 6.3 / 5.7).
+int few_waves(std::size_t tiles) { return tiles >= 512 ? 4 : tiles >= 128 ? 8 : 16; }
 
 // Wavefronts per 64-row tile: each takes about kBlocksPerWave blocks (4 for
 // Q4_0, 2 for Q8_0: about 4 KB of codes and scales in flight per
@@ -842,7 +893,7 @@ int narrow_waves(std::size_t nblk) {
 }
 
 struct TilePlan {
-  int kind = 0;  // 0: the multi-row product (qrows.hip); GroupProblem::kNarrow; or the row chunk R of qgemv_tile
+  int kind = 0;  // 0: the multi-row product (qrows.hip); else a GroupProblem kind
   int waves = 1;
   int bpw = 1;
   std::size_t lds = 0;
@@ -863,13 +914,20 @@ TilePlan plan_single(const DeviceMatrix& m, std::size_t rows) {
     p.lds = narrow_lds(m.in, nblk);
     return p;
   }
-  int r = pick_chunk(rows, nblk, kLdsTarget);
-  if (r == 0) r = pick_chunk(1, nblk, max_lds_per_block());
-  if (r == 0) return p;  // rows too long for LDS staging
-  p.kind = r;
+  if (!wide_fits(nblk)) return p;  // rows too long for LDS staging
+  // Few tiles: 16-row x 16-output tiles spread the product over more CUs
+  // (qrows.hip; 576 x 576 at 4 rows 3.7 us, on 64-row tiles 4.0), which
+  // rows of a partial block take from two rows on (2749 x 1003 4.6, 6.8);
+  // 6 rows and more fill them better (4864 x 896 at 8 rows of Q8_0 5.9, 6.8).
+  if (rows > 1 && nblk <= 64 && m.ntiles <= (rows > 5 ? 128u : 64u) && (rows > 2 || m.in % kBlock != 0)) return p;
+  p.kind = rows == 1 ? 1 : few_kind(m, rows, m.ntiles);
+  if (p.kind == GroupProblem::kFew4 || p.kind == GroupProblem::kFew8) {
+    p.waves = few_waves(m.ntiles);
+    return p;
+  }
   p.bpw = static_cast<int>(ceil_div(nblk, wide_waves(nblk, m.type)));
   p.waves = static_cast<int>(ceil_div(nblk, p.bpw));
-  p.lds = wide_lds(nblk, std::min<std::size_t>(rows, r));
+  p.lds = wide_lds(nblk, std::min<std::size_t>(rows, p.kind));
   return p;
 }
 
@@ -880,6 +938,18 @@ void launch_tile(const DeviceMatrix& m, const float* x, std::size_t rows, const 
   qgemv_tile<TYPE, R><<<grid, static_cast<unsigned>(p.waves * 64), p.lds, s>>>(
       reinterpret_cast<const uint4*>(m.codes), m.scales, x, bias, y, static_cast<int>(m.in), static_cast<int>(m.nblk),
       static_cast<int>(m.out), static_cast<int>(rows), p.bpw, acc);
+}
+
+template <int TYPE, int R>
+void launch_few(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, int acc, int waves,
+                hipStream_t s) {
+  const auto* codes = reinterpret_cast<const uint4*>(m.codes);
+  const unsigned grid = static_cast<unsigned>(m.ntiles);
+  const int in = static_cast<int>(m.in), nblk = static_cast<int>(m.nblk), out = static_cast<int>(m.out);
+  const int nr = static_cast<int>(rows);
+  if (waves == 4) qgemv_few<TYPE, R, 4><<<grid, 256, 0, s>>>(codes, m.scales, x, in, nblk, nr, out, bias, y, acc);
+  else if (waves == 8) qgemv_few<TYPE, R, 8><<<grid, 512, 0, s>>>(codes, m.scales, x, in, nblk, nr, out, bias, y, acc);
+  else qgemv_few<TYPE, R, 16><<<grid, 1024, 0, s>>>(codes, m.scales, x, in, nblk, nr, out, bias, y, acc);
 }
 
 template <int TYPE>
@@ -894,7 +964,8 @@ void launch_typed(const DeviceMatrix& m, const float* x, std::size_t rows, const
     case 1: launch_tile<TYPE, 1>(m, x, rows, bias, y, acc, p, s); break;
     case 2: launch_tile<TYPE, 2>(m, x, rows, bias, y, acc, p, s); break;
     case 4: launch_tile<TYPE, 4>(m, x, rows, bias, y, acc, p, s); break;
-    default: launch_tile<TYPE, 8>(m, x, rows, bias, y, acc, p, s); break;
+    case GroupProblem::kFew4: launch_few<TYPE, 4>(m, x, rows, bias, y, acc, p.waves, s); break;
+    default: launch_few<TYPE, 8>(m, x, rows, bias, y, acc, p.waves, s); break;
   }
 }
 
@@ -950,7 +1021,8 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
   // Products are launched by weight type and row chunk R (one kernel
   // instance each).
   for (int type : {LLMI_TYPE_Q8_0, LLMI_TYPE_Q4_0})
-  for (int R : {int{GroupProblem::kNarrow}, 1, 2, 4, 8}) {
+  for (int R : {int{GroupProblem::kNarrow}, 1, 2, 4, int{GroupProblem::kFew4}, int{GroupProblem::kFew8}}) {
+    const bool few = R == GroupProblem::kFew4 || R == GroupProblem::kFew8;
     std::vector<GroupProblem> probs;
     std::size_t biggest = 0;
     int waves = 1;
@@ -966,9 +1038,8 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
       LLMI_REQUIRE(e.prologue == kPlain || narrow, "group: a prologue needs batch 1 and in <= ~20k");
       LLMI_REQUIRE(e.prologue == kPlain || e.prologue == kRmsNorm || e.prologue == kSiluUp,
                    "group: unknown prologue");
-      int r = narrow ? int{GroupProblem::kNarrow} : pick_chunk(e.rows, m.nblk, kLdsTarget);
-      if (r == 0) r = pick_chunk(1, m.nblk, max_lds_per_block());
-      LLMI_REQUIRE(r != 0, "group: rows too long for the grouped GEMV (in above ~10k)");
+      LLMI_REQUIRE(narrow || wide_fits(m.nblk), "group: rows too long for the grouped GEMV (in above ~10k)");
+      const int r = narrow ? int{GroupProblem::kNarrow} : e.rows == 1 ? 1 : few_kind(m, e.rows, wide_total);
       if (r != R || m.type != type) continue;
       GroupProblem p{};
       p.codes = m.codes;
@@ -1020,9 +1091,11 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
         wgs = ceil_div(p.out, 16);
         need = narrow_lds(p.in, p.nblk);
       } else {
-        p.bpw = static_cast<int>(ceil_div(p.nblk, waves));
-        wgs = static_cast<std::size_t>(p.ntiles) * ceil_div(p.rows, R);
-        need = wide_lds(p.nblk, std::min(p.rows, R));
+        wgs = static_cast<std::size_t>(p.ntiles) * (few ? 1 : ceil_div(p.rows, R));
+        if (!few) {
+          p.bpw = static_cast<int>(ceil_div(p.nblk, waves));
+          need = wide_lds(p.nblk, std::min(p.rows, R));
+        }
       }
       p.first_wg = static_cast<int>(wg);
       wg += wgs;
@@ -1030,6 +1103,7 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
       l.lds = std::max(l.lds, need);
       plan->wg_prob.insert(plan->wg_prob.end(), wgs, static_cast<std::uint32_t>(j));
     }
+    if (few) l.waves = few_waves(wg);
     LLMI_REQUIRE(l.lds <= max_lds_per_block(), "group: a product needs more LDS than one workgroup may use");
     l.total_wgs = static_cast<int>(wg);
     l.nprob = static_cast<int>(probs.size());
@@ -1038,6 +1112,27 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
   }
   return LLMI_OK;
 }
+
+namespace {
+template <int TYPE, int R>
+void launch_group_few_rows(const GroupProblem* probs, const std::uint32_t* map, const GroupLaunch& l, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(l.total_wgs);
+  if (l.waves == 4) qgemv_group_few<TYPE, R, 4><<<grid, 256, 0, s>>>(probs, map);
+  else if (l.waves == 8) qgemv_group_few<TYPE, R, 8><<<grid, 512, 0, s>>>(probs, map);
+  else qgemv_group_few<TYPE, R, 16><<<grid, 1024, 0, s>>>(probs, map);
+}
+template <int TYPE>
+void launch_group_wide(const GroupProblem* probs, const std::uint32_t* map, const GroupLaunch& l, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(l.total_wgs), block = static_cast<unsigned>(l.waves * 64);
+  switch (l.rchunk) {
+    case 1: qgemv_group<TYPE, 1><<<grid, block, l.lds, s>>>(probs, map); break;
+    case 2: qgemv_group<TYPE, 2><<<grid, block, l.lds, s>>>(probs, map); break;
+    case 4: qgemv_group<TYPE, 4><<<grid, block, l.lds, s>>>(probs, map); break;
+    case GroupProblem::kFew4: launch_group_few_rows<TYPE, 4>(probs, map, l, s); break;
+    default: launch_group_few_rows<TYPE, 8>(probs, map, l, s); break;
+  }
+}
+}  // namespace
 
 int launch_group(const GroupProblem* probs_dev, const std::uint32_t* map_dev, const GroupLaunch& l, hipStream_t s) {
   if (l.total_wgs == 0) return LLMI_OK;
@@ -1048,19 +1143,9 @@ int launch_group(const GroupProblem* probs_dev, const std::uint32_t* map_dev, co
     if (l.type == LLMI_TYPE_Q8_0) qgemv_group_narrow<LLMI_TYPE_Q8_0><<<grid, block, l.lds, s>>>(probs, map);
     else qgemv_group_narrow<LLMI_TYPE_Q4_0><<<grid, block, l.lds, s>>>(probs, map);
   } else if (l.type == LLMI_TYPE_Q8_0) {
-    switch (l.rchunk) {
-      case 1: qgemv_group<LLMI_TYPE_Q8_0, 1><<<grid, block, l.lds, s>>>(probs, map); break;
-      case 2: qgemv_group<LLMI_TYPE_Q8_0, 2><<<grid, block, l.lds, s>>>(probs, map); break;
-      case 4: qgemv_group<LLMI_TYPE_Q8_0, 4><<<grid, block, l.lds, s>>>(probs, map); break;
-      default: qgemv_group<LLMI_TYPE_Q8_0, 8><<<grid, block, l.lds, s>>>(probs, map); break;
-    }
+    launch_group_wide<LLMI_TYPE_Q8_0>(probs, map, l, s);
   } else {
-    switch (l.rchunk) {
-      case 1: qgemv_group<LLMI_TYPE_Q4_0, 1><<<grid, block, l.lds, s>>>(probs, map); break;
-      case 2: qgemv_group<LLMI_TYPE_Q4_0, 2><<<grid, block, l.lds, s>>>(probs, map); break;
-      case 4: qgemv_group<LLMI_TYPE_Q4_0, 4><<<grid, block, l.lds, s>>>(probs, map); break;
-      default: qgemv_group<LLMI_TYPE_Q4_0, 8><<<grid, block, l.lds, s>>>(probs, map); break;
-    }
+    launch_group_wide<LLMI_TYPE_Q4_0>(probs, map, l, s);
   }
   LLMI_TRY_HIP(hipGetLastError());
   return LLMI_OK;

@@ -1,6 +1,6 @@
-"""The exact multi-row product (csrc/qrows.hip, more than 8 input rows)
-against the oracle, bit for bit, on the shapes where its tiles and its
-dispatch can go wrong."""
+"""The exact products of more than one input row on the matrix cores
+(csrc/qrows.hip above 8 rows, csrc/qfew.hpp up to 8) against the oracle, bit
+for bit, on the shapes where their tiles and their dispatch can go wrong."""
 
 import numpy as np
 import pytest
@@ -49,20 +49,52 @@ def test_tile_edges_match_oracle(qt, rows, out, n_in):
     assert np.all(got[rows * out :] == 7.0)
 
 
+# 2..8 rows: one side and the other of 4 rows a matrix instruction, of a
+# 64-row tile, of a partial block; 16-row tiles (at most 64 tiles and 64
+# blocks), long rows on few tiles, and 16, 8 and 4 wavefronts per 64-row tile
+# with fewer, as many and more blocks than wavefronts.
+FEW = [(2, 64, 33), (3, 63, 32), (4, 4161, 31), (5, 4200, 32), (8, 4097, 513), (7, 8256, 70), (4, 8192, 288),
+       (3, 32832, 100), (8, 32770, 97), (5, 32768, 160), (2, 32768, 64), (6, 200, 2100), (4, 130, 2048), (3, 8300, 2100)]
+
+
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
-def test_extreme_rows_stay_in_their_rows(qt):
+@pytest.mark.parametrize("rows,out,n_in", FEW)
+def test_few_rows_match_oracle(qt, rows, out, n_in):
+    """Single and grouped; x between values that must not be read as its
+    padding."""
+    orc = O.oracle()
+    w = synth.normal(out + 5 * n_in, out * n_in, 0.0, 0.02)
+    x = synth.normal(rows * 17 + n_in, rows * n_in, 0.0, 1.0)
+    bias = synth.normal(4, out, 0.0, 0.5)
+    data, scales = orc.quantize(w, out, n_in, qt)
+    dev = H.Weight.upload(data, scales, out, n_in, qt)
+    want = orc.matmul(x, rows, n_in, data, scales, qt, out, bias)
+    around = np.full(rows * n_in + 9, np.nan, dtype=np.float32)
+    around[1 : 1 + rows * n_in] = x
+    xd, bd = H.DeviceBuffer.from_array(around), H.DeviceBuffer.from_array(bias)
+    yd = [H.DeviceBuffer.from_array(np.full(rows * out + 64, 7.0, dtype=np.float32)) for _ in range(2)]
+    dev.matmul_dev(xd.ptr + 4, rows, bd.ptr, yd[0].ptr)
+    H.Group([(dev, xd.ptr + 4, yd[1].ptr, rows, bd.ptr)]).launch()
+    H.synchronize()
+    for y in yd:
+        got = y.download(np.float32)
+        assert np.array_equal(bits(got[: rows * out]), bits(want))
+        assert np.all(got[rows * out :] == 7.0)
+
+
+@pytest.mark.parametrize("rows", [5, 24])
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+def test_extreme_rows_stay_in_their_rows(qt, rows):
     """Subnormal, zero, huge and infinite activations: each row's results are
     the oracle's, whatever its neighbours in the tile hold."""
     orc = O.oracle()
-    rows, out, n_in = 24, 80, 96
+    out, n_in = 4500, 96
     w = synth.normal(1, out * n_in, 0.0, 0.02)
     x = synth.normal(2, rows * n_in, 0.0, 1.0).reshape(rows, n_in)
-    x[1] *= np.float32(1e-42)
-    x[2] = 0.0
-    x[3] = -0.0
-    x[4] *= np.float32(1e36)
-    x[5, 7] = np.inf
-    x[6] *= np.float32(1e-30)
+    x[0] *= np.float32(1e-42)
+    x[1] = -0.0
+    x[2] *= np.float32(1e36)
+    x[3, 7] = np.inf
     data, scales = orc.quantize(w, out, n_in, qt)
     scales[::7] *= np.float32(1e-12)
     dev = H.Weight.upload(data, scales, out, n_in, qt)
