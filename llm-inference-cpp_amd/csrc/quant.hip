@@ -1,12 +1,11 @@
 // Block quantizer (fp32 -> Q8_0 / Q4_0), the planar <-> tiled re-layout, and
 // the row dequantizer (embedding gather) for gfx950.
 //
-// The quantizer restates src/model/quant.cpp:36-102 one 32-weight block per
-// thread: the block scan, the scale and every code are computed exactly as
-// the reference computes them (IEEE fp32 divide for the scale, IEEE fp64
-// divide and round-half-away-from-zero for the codes), so the packed bytes
-// are bit-identical.  Load-time work: it reads each weight once (4 B) and
-// writes 0.625 / 1.125 B, so it is HBM-bound.
+// The quantizer restates src/model/quant.cpp:36-102: the block scan, the
+// scale and every code have the reference's values (IEEE fp32 divide for the
+// scale; the codes as its IEEE fp64 divide and round-half-away-from-zero give
+// them), so the packed bytes are bit-identical.  Load-time work: it reads
+// each weight once (4 B) and writes 0.625 / 1.125 B, so it is HBM-bound.
 #include "common.hpp"
 
 namespace llmi_hip {
@@ -23,77 +22,136 @@ __device__ __forceinline__ int round_half_away(double q) {
   return static_cast<int>(r);
 }
 
-template <int TYPE>
-__global__ void __launch_bounds__(256) quantize_blocks(const float* __restrict__ w, std::size_t out, int in, int nblk,
-                                                       std::uint8_t* __restrict__ pdata, float* __restrict__ pscales,
-                                                       std::uint8_t* __restrict__ tcodes,
-                                                       float* __restrict__ tscales) {
-  const std::size_t gid = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= out * static_cast<std::size_t>(nblk)) return;
-  const std::size_t r = gid / nblk;
-  const int b = static_cast<int>(gid % nblk);
-  const int first = b * kBlock;
-  const int n = min(kBlock, in - first);
-  const float* src = w + r * static_cast<std::size_t>(in) + first;
+// The value of a lane's partner within its group of eight lanes: the lane
+// with the lowest bit flipped, the second bit flipped, or (all four lanes of
+// a quad holding one value) a lane of the group's other quad.
+template <int CTRL>
+__device__ __forceinline__ std::uint32_t partner(std::uint32_t v) {
+  return static_cast<std::uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kFlip1 = 0xB1, kFlip2 = 0x4E, kOtherQuad = 0x141;  // quad_perm, quad_perm, row_half_mirror
 
-  float v[kBlock];
-#pragma unroll
-  for (int i = 0; i < kBlock; ++i) v[i] = i < n ? src[i] : 0.0f;
-
-  // quant.cpp:54-62: strict '>' keeps the first index of the largest |v|.
-  float peak = 0.0f, peak_signed = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kBlock; ++i) {
-    const float mag = fabsf(v[i]);
-    if (i < n && mag > peak) {
-      peak = mag;
-      peak_signed = v[i];
-    }
+// The reference's code lround(double(v) / double(d)) (quant.cpp:85), without
+// the double division where its rounding is not in doubt.  r is 1 / d within
+// an ulp, so |v * r| is within 2^-15 of |v / d| <= 128; unless it lies within
+// kDoubt of a half it rounds to the same integer.  (The double quotient is a
+// half exactly when the real one is: v / d - (n + 1/2) is 0 or, for fp32 v
+// and d and n < 128, at least 2^-25.)
+constexpr float kDoubt = 0x1p-13f;
+__device__ __forceinline__ int code_of_value(float v, float d, float r, bool fast) {
+  const float a = v * r;
+  const float m = __builtin_fabsf(a) + 0.5f;
+  const float f = __builtin_floorf(m);
+  const float frac = m - f;
+  if (fast && frac >= kDoubt && frac <= 1.0f - kDoubt) {
+    const int n = static_cast<int>(f);
+    return a < 0.0f ? -n : n;
   }
-  float d = TYPE == LLMI_TYPE_Q4_0 ? peak_signed / -8.0f : peak / 127.0f;  // quant.cpp:63-80
-  if (d == 0.0f) d = 1.0f;                                                  // quant.cpp:81
-  const int hi = TYPE == LLMI_TYPE_Q4_0 ? 7 : 127;
-  const int lo = TYPE == LLMI_TYPE_Q4_0 ? -8 : -127;
+  return round_half_away(static_cast<double>(v) / static_cast<double>(d));
+}
 
-  // Codes, packed into 32-bit words in the reference's byte order.
-  constexpr int kWords = TYPE == LLMI_TYPE_Q4_0 ? 4 : 8;
-  std::uint32_t word[kWords];
+typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Eight lanes per (row, block), four weights each: a block is one coalesced
+// 128-byte read, its largest weight three lane exchanges.  The blocks come in
+// the order of the output -- planar: by row; tiled: the 64 rows of a tile one
+// after another, block by block -- so that the codes of consecutive groups
+// are neighbours.  Bound: HBM.  Measured on the 151936 x 896 matrix, against
+// one thread per block, whose 128-byte-strided loads and 32 double divisions
+// it replaces: Q4_0 355 -> 125 us (5.0 TB/s).
+constexpr int kQuantItems = 4;  // blocks per group, their loads issued together
+
+template <int TYPE, bool PLANAR>
+__global__ void __launch_bounds__(256) quantize_blocks(const float* __restrict__ w, std::size_t out, int in, int nblk,
+                                                       std::uint8_t* __restrict__ codes, float* __restrict__ scales) {
+  const int tid = threadIdx.x, e0 = 4 * (tid & 7), group = tid >> 3;
+  const bool whole = in % kBlock == 0;
+  float v[kQuantItems][4];
+  std::size_t row[kQuantItems];
+  int block[kQuantItems];
+  // Blocks past the last are not stored; they read the last row's.
 #pragma unroll
-  for (int k = 0; k < kWords; ++k) word[k] = 0u;
+  for (int u = 0; u < kQuantItems; ++u) {
+    const std::size_t item = (static_cast<std::size_t>(blockIdx.x) * kQuantItems + u) * 32 + group;
+    if (PLANAR) {
+      row[u] = item / nblk;
+      block[u] = static_cast<int>(item - row[u] * nblk);
+    } else {
+      const std::size_t slot = (static_cast<std::size_t>(blockIdx.x) * kQuantItems + u) / 2;  // (uniform)
+      row[u] = slot / nblk * kTileRows + (item & (kTileRows - 1));
+      block[u] = static_cast<int>(slot % nblk);
+    }
+    const std::size_t r = row[u] < out ? row[u] : out - 1;
+    const float* src = w + r * static_cast<std::size_t>(in) + block[u] * kBlock;
+    if (whole) {
+      const f32x4a4 x = *reinterpret_cast<const f32x4a4*>(src + e0);
 #pragma unroll
-  for (int i = 0; i < kBlock; ++i) {
-    if (i < n) {
-      int q = round_half_away(static_cast<double>(v[i]) / static_cast<double>(d));  // quant.cpp:85
-      q = min(max(q, lo), hi);
-      if (TYPE == LLMI_TYPE_Q8_0) {
-        word[i / 4] |= (static_cast<std::uint32_t>(q) & 0xFFu) << (8 * (i % 4));
-      } else {
-        word[i / 8] |= static_cast<std::uint32_t>(q + 8) << (4 * (i % 8));
+      for (int e = 0; e < 4; ++e) v[u][e] = x[e];
+    } else {
+      const int n = in - block[u] * kBlock;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = src[min(e0 + e, n - 1)];
+        v[u][e] = e0 + e < n ? x : 0.0f;
       }
     }
   }
-
-  if (pdata != nullptr) {
-    const std::size_t rb = TYPE == LLMI_TYPE_Q4_0 ? (static_cast<std::size_t>(in) + 1) / 2 : static_cast<std::size_t>(in);
-    std::uint8_t* dst = pdata + r * rb + (TYPE == LLMI_TYPE_Q4_0 ? first / 2 : first);
-    const int nbytes = TYPE == LLMI_TYPE_Q4_0 ? (n + 1) / 2 : n;
 #pragma unroll
-    for (int j = 0; j < (TYPE == LLMI_TYPE_Q4_0 ? 16 : 32); ++j)
-      if (j < nbytes) dst[j] = static_cast<std::uint8_t>(word[j / 4] >> (8 * (j % 4)));
-    pscales[r * nblk + b] = d;
-  }
-  if (tcodes != nullptr) {
-    const std::size_t tile = r / kTileRows;
-    const int lane = static_cast<int>(r % kTileRows);
-    const std::size_t slot = tile * nblk + b;
-    if (TYPE == LLMI_TYPE_Q4_0) {
-      reinterpret_cast<uint4*>(tcodes)[slot * kTileRows + lane] = make_uint4(word[0], word[1], word[2], word[3]);
-    } else {
-      uint4* dst = reinterpret_cast<uint4*>(tcodes);
-      dst[(slot * 2 + 0) * kTileRows + lane] = make_uint4(word[0], word[1], word[2], word[3]);
-      dst[(slot * 2 + 1) * kTileRows + lane] = make_uint4(word[4], word[5], word[6], word[7]);
+  for (int u = 0; u < kQuantItems; ++u) {
+    // quant.cpp:54-62: the first of the largest |v| (strict '>': NaN never).
+    float peak = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (__builtin_fabsf(v[u][e]) > __builtin_fabsf(peak)) peak = v[u][e];
+    const auto merge = [&](float other, bool lower) {
+      const float a = __builtin_fabsf(peak), b = __builtin_fabsf(other);
+      if (b > a || (b == a && lower)) peak = other;
+    };
+    merge(__uint_as_float(partner<kFlip1>(__float_as_uint(peak))), (tid & 1) != 0);
+    merge(__uint_as_float(partner<kFlip2>(__float_as_uint(peak))), (tid & 2) != 0);
+    merge(__uint_as_float(partner<kOtherQuad>(__float_as_uint(peak))), (tid & 4) != 0);
+    float d = TYPE == LLMI_TYPE_Q4_0 ? peak / -8.0f : __builtin_fabsf(peak) / 127.0f;  // quant.cpp:63-80
+    if (d == 0.0f) d = 1.0f;                                                           // quant.cpp:81
+    const float size = __builtin_fabsf(d);
+    const bool fast = size >= 0x1p-100f && size <= 0x1p100f;  // 1 / d and v / d are normal numbers
+    const float r = __builtin_amdgcn_rcpf(d);
+    const int left = whole ? kBlock : in - block[u] * kBlock - e0;
+    std::uint32_t word = 0u;  // the four codes, in the reference's byte order
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int q = min(max(code_of_value(v[u][e], d, r, fast), TYPE == LLMI_TYPE_Q4_0 ? -8 : -127),
+                        TYPE == LLMI_TYPE_Q4_0 ? 7 : 127);
+      const std::uint32_t c = TYPE == LLMI_TYPE_Q8_0 ? static_cast<std::uint32_t>(q) & 0xFFu
+                                                     : static_cast<std::uint32_t>(q + 8);
+      word |= (e < left ? c : 0u) << ((TYPE == LLMI_TYPE_Q8_0 ? 8 : 4) * e);
     }
-    tscales[slot * kTileRows + lane] = d;
+    // Q4_0: two lanes make a word, stored by the even one.
+    if (TYPE == LLMI_TYPE_Q4_0) word |= partner<kFlip1>(word) << 16;
+    if (row[u] >= out) continue;
+    const bool first = (tid & 7) == 0;
+    if (PLANAR) {
+      const std::size_t rb = TYPE == LLMI_TYPE_Q4_0 ? (static_cast<std::size_t>(in) + 1) / 2 : static_cast<std::size_t>(in);
+      std::uint8_t* dst = codes + row[u] * rb + (block[u] * kBlock + e0) / (TYPE == LLMI_TYPE_Q4_0 ? 2 : 1);
+      if (whole && reinterpret_cast<std::uintptr_t>(codes) % 4 == 0) {
+        if (TYPE == LLMI_TYPE_Q8_0 || (tid & 1) == 0) *reinterpret_cast<std::uint32_t*>(dst) = word;
+      } else {
+        const int nbytes = TYPE == LLMI_TYPE_Q4_0 ? (min(left, 4) + 1) / 2 : min(left, 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j < nbytes) dst[j] = static_cast<std::uint8_t>(word >> (8 * j));
+      }
+      if (first) scales[row[u] * nblk + block[u]] = d;
+    } else {
+      const std::size_t item = (static_cast<std::size_t>(blockIdx.x) * kQuantItems + u) * 32 + group;  // slot * 64 + row
+      if (TYPE == LLMI_TYPE_Q4_0) {
+        if ((tid & 1) == 0) *reinterpret_cast<std::uint32_t*>(codes + item * 16 + e0 / 2) = word;
+      } else {
+        const std::size_t slot = item / kTileRows, lane = item % kTileRows;
+        *reinterpret_cast<std::uint32_t*>(codes + ((slot * 2 + e0 / 16) * kTileRows + lane) * 16 + e0 % 16) = word;
+      }
+      if (first) scales[item] = d;
+    }
   }
 }
 
@@ -273,15 +331,20 @@ unsigned grid_for(std::size_t work, unsigned threads) { return static_cast<unsig
 int launch_quantize(const float* w, std::size_t out, std::size_t in, int type, std::uint8_t* planar_data,
                     float* planar_scales, DeviceMatrix* tiled, hipStream_t s) {
   const int nblk = static_cast<int>(ceil_div(in, kBlock));
-  const std::size_t work = out * static_cast<std::size_t>(nblk);
+  const std::size_t rows = tiled != nullptr ? ceil_div(out, kTileRows) * kTileRows : out;
+  const std::size_t work = rows * static_cast<std::size_t>(nblk);
   if (work == 0) return LLMI_OK;
-  std::uint8_t* tc = tiled != nullptr ? tiled->codes : nullptr;
-  float* ts = tiled != nullptr ? tiled->scales : nullptr;
-  const unsigned g = grid_for(work, 256);
-  if (type == LLMI_TYPE_Q8_0) {
-    quantize_blocks<LLMI_TYPE_Q8_0><<<g, 256, 0, s>>>(w, out, static_cast<int>(in), nblk, planar_data, planar_scales, tc, ts);
+  const unsigned g = grid_for(work, 32 * kQuantItems);
+  const int n = static_cast<int>(in);
+  if (tiled != nullptr) {
+    if (type == LLMI_TYPE_Q8_0)
+      quantize_blocks<LLMI_TYPE_Q8_0, false><<<g, 256, 0, s>>>(w, out, n, nblk, tiled->codes, tiled->scales);
+    else
+      quantize_blocks<LLMI_TYPE_Q4_0, false><<<g, 256, 0, s>>>(w, out, n, nblk, tiled->codes, tiled->scales);
+  } else if (type == LLMI_TYPE_Q8_0) {
+    quantize_blocks<LLMI_TYPE_Q8_0, true><<<g, 256, 0, s>>>(w, out, n, nblk, planar_data, planar_scales);
   } else {
-    quantize_blocks<LLMI_TYPE_Q4_0><<<g, 256, 0, s>>>(w, out, static_cast<int>(in), nblk, planar_data, planar_scales, tc, ts);
+    quantize_blocks<LLMI_TYPE_Q4_0, true><<<g, 256, 0, s>>>(w, out, n, nblk, planar_data, planar_scales);
   }
   LLMI_TRY_HIP(hipGetLastError());
   return LLMI_OK;
