@@ -103,3 +103,35 @@ def test_extreme_rows_stay_in_their_rows(qt, rows):
     nan = np.isnan(want)
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(bits(got)[~nan], bits(want)[~nan])
+
+
+# fp32 weights (csrc/f32.hip): 16- and 32-row tiles of the matrix-core form,
+# outputs around its 64- and 32-output tiles, elements around a 64-element
+# step, a 16-element chunk and the scalar rest.
+@pytest.mark.parametrize("rows,out,n_in", [(2, 40000, 500), (16, 8001, 64), (16, 5000, 79), (17, 3000, 128),
+                                           (32, 2911, 255), (33, 1600, 1003), (70, 1100, 16), (5, 90000, 31)])
+def test_f32_rows_match_single_rows_and_oracle(rows, out, n_in):
+    """Every output against the one-row product (tests/test_gpu_f32.py holds
+    that one to the oracle), some of them against the oracle's dot."""
+    orc = O.oracle()
+    w = synth.normal(out + 3 * n_in, out * n_in, 0.0, 0.02)
+    x = synth.normal(rows + n_in, rows * n_in, 0.0, 1.0)
+    x[: n_in // 2] *= np.float32(1e-30)  # products that underflow to either zero
+    w[: n_in // 2] *= np.float32(-1e-16)
+    bias = synth.normal(6, out, 0.0, 0.5)
+    bias[::5] = -0.0
+    dev = H.Weight.quantize(w, out, n_in, H.F32)
+    around = np.full(rows * n_in + 9, np.nan, dtype=np.float32)
+    around[1 : 1 + rows * n_in] = x
+    xd, bd = H.DeviceBuffer.from_array(around), H.DeviceBuffer.from_array(bias)
+    yd = H.DeviceBuffer.from_array(np.full(rows * out + 64, 7.0, dtype=np.float32))
+    dev.matmul_dev(xd.ptr + 4, rows, bd.ptr, yd.ptr)
+    H.synchronize()
+    got = yd.download(np.float32)
+    want = np.concatenate([dev.matmul(x[r * n_in : (r + 1) * n_in], 1, bias) for r in range(rows)])
+    assert np.array_equal(bits(got[: rows * out]), bits(want))
+    for i in np.random.default_rng(n_in).integers(0, rows * out, 60):
+        r, o = divmod(int(i), out)
+        d = np.float32(orc.dot(x[r * n_in : (r + 1) * n_in], w[o * n_in : (o + 1) * n_in])) + bias[o]
+        assert bits(got[i : i + 1])[0] == bits(np.float32([d]))[0]
+    assert np.all(got[rows * out :] == 7.0)
