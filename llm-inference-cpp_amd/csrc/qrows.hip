@@ -114,10 +114,18 @@ __device__ __forceinline__ void lane_codes(const Block<TYPE>& b, int q, float* c
       c[i + 1] = static_cast<float>(static_cast<std::int8_t>((v >> 8) & 0xFFu));
     }
   } else {
-    std::uint32_t w[8];
-    unpack_words<TYPE>(b, w);
+    // Nibbles q and q + 4 of words j and j + 1: their bytes side by side,
+    // the nibbles as signed bytes n - 8 (n + 0x78 never carries out of its
+    // byte), then converted by byte.
+    const std::uint32_t sel = 0x06040200u + 0x01010101u * static_cast<std::uint32_t>(q >> 1);
+    const std::uint32_t w[4] = {b.c[0].x, b.c[0].y, b.c[0].z, b.c[0].w};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) c[i] = static_cast<float>(sfield(w[i >> 1], 4 * q + 16 * (i & 1), 4));
+    for (int j = 0; j < 4; j += 2) {
+      const std::uint32_t t = __builtin_amdgcn_perm(w[j + 1], w[j], sel) >> (4 * (q & 1));
+      const std::uint32_t v = ((t & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[2 * j + e] = static_cast<float>(static_cast<std::int8_t>(v >> (8 * e)));
+    }
   }
 }
 
@@ -129,7 +137,7 @@ __device__ __forceinline__ void lane_codes(const Block<TYPE>& b, int q, float* c
 // A 32-bit lane offset that stays one: widened inside the loop (by the load's
 // own addressing mode) instead of once before it, where it would cost a
 // 64-bit vector addition per load.
-__device__ __forceinline__ std::uint32_t opaque(std::uint32_t v) {
+__device__ __forceinline__ std::uint32_t opaque(std::uint32_t& v) {
   asm("" : "+v"(v));
   return v;
 }
@@ -151,6 +159,7 @@ struct RowsTile {
   const GMEM char* sb;
   float* xs;                     // [16 * TT][kRowStride]
   int in, n, q, lane, sub;
+  std::uint32_t co, so;  // lane offsets of the codes and scales, in bytes
 
   // Rows past the last are the last one again (computed, never stored).
   __device__ __forceinline__ void init(const float* x, int in_, int rows, int r0, int lane_, float* lds) {
@@ -172,8 +181,10 @@ struct RowsTile {
     cb = reinterpret_cast<const GMEM char*>(gmem(codes) + base * Block<TYPE>::kU);
     sb = reinterpret_cast<const GMEM char*>(gmem(scales) + base);
     sub = sub_;
+    co = 16u * sub;
+    so = 4u * sub;
   }
-  __device__ __forceinline__ void load(Raw& r, int b) const {
+  __device__ __forceinline__ void load(Raw& r, int b) {
     const GMEM char* p = xb + static_cast<std::size_t>(b) * kBlock * 4;
     if (WHOLE || b < in / kBlock) {  // (uniform) four elements at once; a row need only be 4-byte aligned
 #pragma unroll
@@ -192,10 +203,10 @@ struct RowsTile {
     const GMEM char* c = cb + static_cast<std::size_t>(b) * (kTileRows * 16 * Block<TYPE>::kU);
 #pragma unroll
     for (int u = 0; u < Block<TYPE>::kU; ++u) {
-      const u32x4 v = *reinterpret_cast<const GMEM u32x4*>(c + opaque(16u * sub) + u * (kTileRows * 16u));
+      const u32x4 v = *reinterpret_cast<const GMEM u32x4*>(c + opaque(co) + u * (kTileRows * 16u));
       r.blk.c[u] = uint4{v.x, v.y, v.z, v.w};
     }
-    r.sc = *reinterpret_cast<const GMEM float*>(sb + static_cast<std::size_t>(b) * (kTileRows * 4) + opaque(4u * sub));
+    r.sc = *reinterpret_cast<const GMEM float*>(sb + static_cast<std::size_t>(b) * (kTileRows * 4) + opaque(so));
   }
   // Element 4i + e of the block goes to [e][i].  Activations past `in` (the
   // last block's) become zero: the codes stored there then add nothing.
