@@ -21,12 +21,16 @@
 // passes are rare (a threshold within ~1e-11 relative of a running sum).
 //
 // Kernels of one sampling call (temperature > 0), all on one stream:
-//   smp_max    max of logits / temperature (float division), NaN / +inf flags
-//   smp_exp    e = expf(x / T - max) (the exact expf), sum -> inv = float(1/sum)
+//   smp_max    each slice's max of logits / temperature (float division),
+//              NaN / +inf flags
+//   smp_exp    e = expf(x / T - max) (the exact expf), each slice's sum and
+//              largest e
 //   when 0 < top_k <= kSelectMax (the ranking's first k):
-//     smp_sel_local  p = e * inv; each slice's first k, in index order
+//     smp_sel_local  inv = float(1/sum), p = e * inv; each slice's entries that
+//                    can be among the ranking's first k, in index order
 //     smp_sel_merge  the first k among those, ranked
-//   else, when something is filtered (the whole ranking):
+//   else smp_exp's last workgroup takes inv, and when something is filtered
+//   (the whole ranking):
 //     smp_scale  p = e * inv and the ranking keys (float bits, index)
 //     smp_sort_hist / smp_sort_scan / smp_sort_scatter, four times: the
 //                ranking by a stable LSD radix sort (descending p, ties in
@@ -82,7 +86,7 @@ struct SmpWork {
   std::int32_t* idx;
   std::int32_t* idx_sorted;
   double* part_d;            // per-block partials
-  int* part_i;
+  int* part_i;               // (the upper half: smp_exp's largest e of each slice, as bits)
   float* part_f;
   SmpState* st;
 };
@@ -313,72 +317,111 @@ __device__ int block_sequential_sum(F v, int m, bool has_stop, double stop_at, d
 }
 
 // ------------------------------------------------------------------ kernels
-__global__ void __launch_bounds__(kSmpThreads) smp_max(const float* __restrict__ logits, int n, float temp, SmpWork w,
-                                                       SampleLog* __restrict__ log) {
+// The grid of a sampling call is one or two waves per SIMD on half the chip,
+// so its kernels are bound by dependent memory round trips and barriers, not
+// by the logits' bytes (608 KB of fp32 at 151,936 entries).  Hence: a slice's
+// entries are read kHeld per thread at a time, every load issued before the
+// first use, and what one kernel's workgroups find (a partial per slice) is
+// combined by each wave of the next kernel's workgroups rather than by the
+// last workgroup of the same launch, whose atomic, barrier and second read of
+// the partials took ~3 us a kernel.  On 151,936 logits, top-k 40: smp_max 8.0 ->
+// 3.3 us, smp_exp 11.3 -> 4.3, smp_sel_local 10.4 -> 4.1 and smp_sel_merge 20 ->
+// 10.3 (with the candidate bound below), a call 66.7 -> 42.2 us.
+constexpr int kHeld = 8;
+
+// fn(i, src[i]) for this thread's entries of the slice; each round's loads
+// are issued together.
+template <typename F>
+__device__ __forceinline__ void for_slice(const float* src, Slice sl, F fn) {
+  for (int c0 = sl.lo; c0 < sl.hi; c0 += kHeld * kSmpThreads) {
+    const int i0 = c0 + static_cast<int>(threadIdx.x);
+    float x[kHeld];
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q) x[q] = src[min(i0 + q * kSmpThreads, sl.hi - 1)];
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q) {
+      const int i = i0 + q * kSmpThreads;
+      if (i < sl.hi) fn(i, x[q]);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kSmpThreads) smp_max(const float* __restrict__ logits, int n, float temp, SmpWork w) {
   __shared__ float red_f[kSmpWaves];
   __shared__ int red_i[kSmpWaves];
-  __shared__ bool last;
-  const Slice sl = slice_of(n, blockIdx.x, gridDim.x);
   float m = -__builtin_inff();
   int fl = 0;
-  for (int i = sl.lo + static_cast<int>(threadIdx.x); i < sl.hi; i += kSmpThreads) {
-    const float v = logits[i] / temp;
+  for_slice(logits, slice_of(n, blockIdx.x, gridDim.x), [&](int, float x) {
+    const float v = x / temp;
     if (v != v) fl |= kFlagNaN;
     if (v == __builtin_inff()) fl |= kFlagPosInf;
     m = fmaxf(m, v);
-  }
+  });
   m = block_max_f(m, red_f);
   fl = block_or(fl, red_i);
   if (threadIdx.x == 0) {
     w.part_f[blockIdx.x] = m;
     w.part_i[blockIdx.x] = fl;
-    last = arrive_last(&w.st->counter);
-  }
-  __syncthreads();
-  if (!last) return;
-  float mm = -__builtin_inff();
-  int ff = 0;
-  for (int b = threadIdx.x; b < static_cast<int>(gridDim.x); b += kSmpThreads) {
-    mm = fmaxf(mm, load_relaxed(w.part_f + b));
-    ff |= load_relaxed(w.part_i + b);
-  }
-  mm = block_max_f(mm, red_f);
-  ff = block_or(ff, red_i);
-  if (threadIdx.x == 0) {
-    if (ff == 0 && mm == -__builtin_inff()) ff = kFlagAllNegInf;
-    w.st->mx = mm;
-    w.st->flags = ff;
-    w.st->seq_paths = 0;
-    w.st->decided = 0;
-    if (log != nullptr) *log = SampleLog{-1, ff << 1};  // smp_draw overwrites it when it decides
-    reset_counter(&w.st->counter);
   }
 }
 
-// kernels.cpp:136-146 on x / temperature.
-__global__ void __launch_bounds__(kSmpThreads) smp_exp(const float* __restrict__ logits, int n, float temp, SmpWork w) {
+// The exact softmax denominator decides inv where the bound on its parallel
+// sum leaves float(1/sum) open: its terms recomputed from the logits.
+__device__ __forceinline__ float sequential_inv(const float* __restrict__ logits, int n, float temp, float mx,
+                                                const std::uint64_t* tab, double* seq, float* stage, int* stop) {
+  block_sequential_sum([=](int j) { return exact::expf_with(logits[j] / temp - mx, tab); }, n, false, 0.0, seq, stage,
+                       stop);
+  return recip_float(*seq);
+}
+
+// kernels.cpp:136-146 on x / temperature.  With `finish` the last workgroup
+// combines the slices' sums; else smp_sel_local does.
+static_assert(kSmpBlocks == 128, "a lane combines two slices' partials");
+__global__ void __launch_bounds__(kSmpThreads) smp_exp(const float* __restrict__ logits, int n, float temp, int finish,
+                                                       SmpWork w, SampleLog* __restrict__ log) {
   __shared__ std::uint64_t tab[32];
   __shared__ double red_d[kSmpWaves];
+  __shared__ float red_f[kSmpWaves];
   __shared__ float stage[2 * kSeqChunk];
   __shared__ int stop[2];
   __shared__ double seq;
   __shared__ bool last;
-  if (w.st->flags & kFlagBad) return;
+  const int l = threadIdx.x & 63;
+  const float m0 = w.part_f[l], m1 = w.part_f[l + 64];
+  const int f01 = w.part_i[l] | w.part_i[l + 64];
   if (threadIdx.x < 32) tab[threadIdx.x] = exact::kExp2Tab[threadIdx.x];
+  const float mx = wave_max_dpp(fmaxf(m0, m1));
+  int flags = (__builtin_amdgcn_ballot_w64((f01 & kFlagNaN) != 0) != 0 ? kFlagNaN : 0) |
+              (__builtin_amdgcn_ballot_w64((f01 & kFlagPosInf) != 0) != 0 ? kFlagPosInf : 0);
+  if (flags == 0 && mx == -__builtin_inff()) flags = kFlagAllNegInf;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    w.st->mx = mx;
+    w.st->flags = flags;
+    w.st->seq_paths = 0;
+    w.st->decided = 0;
+    if (log != nullptr) *log = SampleLog{-1, flags << 1};  // smp_draw overwrites it when it decides
+  }
+  if (flags & kFlagBad) return;
   __syncthreads();
-  const float mx = w.st->mx;
   const Slice sl = slice_of(n, blockIdx.x, gridDim.x);
   double part = 0.0;
-  for (int i = sl.lo + static_cast<int>(threadIdx.x); i < sl.hi; i += kSmpThreads) {
-    const float e = exact::expf_with(logits[i] / temp - mx, tab);
+  float top = 0.0f;
+  for_slice(logits, sl, [&](int i, float x) {
+    const float e = exact::expf_with(x / temp - mx, tab);
     w.p[i] = e;
     part = part + static_cast<double>(e);
-  }
+    top = fmaxf(top, e);
+  });
+  top = wave_max_dpp(top);
+  if (l == 0) red_f[threadIdx.x >> 6] = top;
   part = block_sum_d(part, red_d);
   if (threadIdx.x == 0) {
+    for (int q = 1; q < kSmpWaves; ++q) top = fmaxf(top, red_f[q]);
     w.part_d[blockIdx.x] = part;
-    last = arrive_last(&w.st->counter);
+    w.part_i[kSmpBlocks + blockIdx.x] = __builtin_bit_cast(int, top);
   }
+  if (!finish) return;
+  if (threadIdx.x == 0) last = arrive_last(&w.st->counter);
   __syncthreads();
   if (!last) return;
   __shared__ float inv_s;
@@ -392,11 +435,7 @@ __global__ void __launch_bounds__(kSmpThreads) smp_exp(const float* __restrict__
   __syncthreads();
   float inv = inv_s;
   if (inv < 0.0f) {
-    // The bound leaves float(1/sum) open: the sequential sum, its terms
-    // recomputed from the logits (other workgroups' e need not be visible).
-    block_sequential_sum([=](int j) { return exact::expf_with(logits[j] / temp - mx, tab); }, n, false, 0.0, &seq,
-                         stage, stop);
-    inv = recip_float(seq);
+    inv = sequential_inv(logits, n, temp, mx, tab, &seq, stage, stop);
     if (threadIdx.x == 0) w.st->seq_paths |= kSeqSoftmax;
   }
   if (threadIdx.x == 0) {
@@ -492,15 +531,26 @@ __device__ __forceinline__ float renorm(float p, double s) {
 // The first k entries of the ranking (p descending, equal p by index, the
 // order std::stable_sort gives sampling.cpp:30-34) without sorting all n, for
 // 0 < top_k <= kSelectMax.  Keys are the bits of p = e * inv (p >= +0, so
-// their unsigned order is p's order); a select finds the k-th largest key K
-// by four 8-bit radix passes over LDS histograms (integer counts: every
-// decision is exact) and keeps every key above K and the lowest-index entries
-// equal to it.  smp_sel_local does that per slice, writing the slice's first
-// k in index order; the ranking's first k are among those candidates, which
-// are then in index order overall, and smp_sel_merge selects again over them
-// and ranks the k it keeps.
+// their unsigned order is p's order).  If k slices have a largest p of at
+// least T, so has the ranking's k-th entry: only entries >= T can be among
+// the first k (p = float(e * inv) never falls as e grows, so the bound may be
+// taken from the slices' largest e).  T is found in each wave by a binary
+// search with two ballots a step, on the top 16 bits (a bf16 below the k-th
+// largest: a little lower, so still a bound).  On scattered logits about k
+// entries of the whole vocabulary pass, and smp_sel_merge ranks them by
+// counting.  Where more than kSelectMax of a slice pass (equal or clustered
+// logits, or fewer than k slices that hold any), smp_sel_local selects the
+// slice's first k: the k-th largest key K by four 8-bit radix passes over LDS
+// histograms (integer counts: every decision is exact), every key above K and
+// the lowest-index entries equal to it.  Either way a slice's candidates are
+// in index order, hence all of them; and where more than kDirectMax are left,
+// smp_sel_merge does the same radix select over them before it ranks.  (The
+// radix select over 128 * k candidates was most of smp_sel_merge's 20 us:
+// twelve barriers of 16 waves, and LDS atomics on the few bins that the
+// largest probabilities share.)
 constexpr int kSelectMax = 64;
 constexpr int kCandMax = kSmpBlocks * kSelectMax;
+constexpr int kDirectMax = 256;  // candidates ranked by counting alone
 static_assert(kSmpThreads == 256, "one histogram bin per thread");
 
 __device__ __forceinline__ std::uint32_t key_bits(float p) { return __builtin_bit_cast(std::uint32_t, p); }
@@ -558,50 +608,106 @@ __device__ __forceinline__ int block_count_prefix(int v, int* wave_tot, int* tot
   return r;
 }
 
-// Scales the slice (p = e * inv, the work of smp_scale) and writes its first
-// min(k, slice) entries of the ranking, in index order, to
-// keys / idx [b * kSelectMax, ...); their count to part_i[b].
-__global__ void __launch_bounds__(kSmpThreads) smp_sel_local(int n, int k, SmpWork w) {
+// Scales the slice (p = e * inv, the work of smp_scale) and writes its
+// candidates, in index order, to keys / idx [b * kSelectMax, ...); their count
+// to part_i[b].
+__global__ void __launch_bounds__(kSmpThreads) smp_sel_local(const float* __restrict__ logits, int n, float temp, int k,
+                                                             SmpWork w) {
   __shared__ int hist[256];
   __shared__ unsigned sel[2];
   __shared__ int wave_tot[kSmpWaves];
-  if (w.st->flags & kFlagBad) return;
+  __shared__ int slot;
+  __shared__ std::uint32_t ck[kSelectMax];
+  __shared__ std::int32_t ci[kSelectMax];
+  const int t = threadIdx.x, l = t & 63;
+  const double d0 = w.part_d[l], d1 = w.part_d[l + 64];
+  const std::uint32_t e0 = static_cast<std::uint32_t>(w.part_i[kSmpBlocks + l]);
+  const std::uint32_t e1 = static_cast<std::uint32_t>(w.part_i[kSmpBlocks + l + 64]);
+  const int flags = w.st->flags;
   const Slice sl = slice_of(n, blockIdx.x, gridDim.x);
-  const int want = min(k, sl.hi - sl.lo);
-  const int t = threadIdx.x;
-  const float inv = w.st->inv;
   if (t == 0) {
     sel[0] = 0u;
     sel[1] = 0u;
+    slot = 0;
   }
+  __syncthreads();
+  if (flags & kFlagBad) return;
+  const double sum = wave_sum(d0 + d1);  // the same in every wave: one tree
+  const double slack = smp_sigma(n) * sum;
+  float inv = recip_float(sum - slack);
+  if (inv != recip_float(sum + slack)) {  // (the same in every workgroup)
+    __shared__ std::uint64_t tab[32];
+    __shared__ float stage[2 * kSeqChunk];
+    __shared__ int stop[2];
+    __shared__ double seq;
+    if (t < 32) tab[t] = exact::kExp2Tab[t];
+    __syncthreads();
+    inv = sequential_inv(logits, n, temp, w.st->mx, tab, &seq, stage, stop);
+    if (blockIdx.x == 0 && t == 0) w.st->seq_paths |= kSeqSoftmax;
+  }
+  if (blockIdx.x == 0 && t == 0) w.st->inv = inv;
+  std::uint32_t bound = 0;
+#pragma unroll
+  for (int bit = 29; bit >= 16; --bit) {  // e <= 1: bit 30 is never set
+    const std::uint32_t c = bound | (1u << bit);
+    const int cnt = __builtin_popcountll(__builtin_amdgcn_ballot_w64(e0 >= c)) +
+                    __builtin_popcountll(__builtin_amdgcn_ballot_w64(e1 >= c));
+    if (cnt >= k) bound = c;
+  }
+  const float p_min = __builtin_bit_cast(float, bound) * inv;
+  for_slice(w.p, sl, [&](int i, float e) {
+    const float p = e * inv;
+    w.p[i] = p;
+    if (p >= p_min) {
+      const int q = atomicAdd(&slot, 1);
+      if (q < kSelectMax) {
+        ck[q] = key_bits(p);
+        ci[q] = i;
+      }
+    }
+  });
+  __syncthreads();
+  std::uint32_t* keys = w.keys + blockIdx.x * kSelectMax;
+  std::int32_t* idx = w.idx + blockIdx.x * kSelectMax;
+  const int passed = slot;
+  if (passed <= kSelectMax) {
+    if (t < 64) {
+      const std::uint32_t kt = t < passed ? ck[t] : 0u;
+      const std::int32_t it = t < passed ? ci[t] : 0;
+      int better = 0;  // only the slice's first k: tied logits pass in numbers
+      if (passed > k)
+        for (int q = 0; q < passed; ++q) better += (ck[q] > kt || (ck[q] == kt && ci[q] < it)) ? 1 : 0;
+      const unsigned long long in = __builtin_amdgcn_ballot_w64(t < passed && better < k);
+      int pos = 0;
+      for (int q = 0; q < passed; ++q) pos += ((in >> q) & 1) != 0 && ci[q] < it ? 1 : 0;
+      if ((in >> t) & 1) {
+        keys[pos] = kt;
+        idx[pos] = it;
+      }
+    }
+    if (t == 0) w.part_i[blockIdx.x] = min(passed, k);
+    return;
+  }
+  const int want = min(k, sl.hi - sl.lo);
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
     hist[t] = 0;
     __syncthreads();
     const unsigned prefix = sel[0];
     for (int i = sl.lo + t; i < sl.hi; i += kSmpThreads) {
-      std::uint32_t key;
-      if (pass == 0) {
-        const float p = w.p[i] * inv;
-        w.p[i] = p;
-        key = key_bits(p);
-      } else {
-        key = key_bits(w.p[i]);
-      }
+      const std::uint32_t key = key_bits(w.p[i]);
       if (pass == 0 || (key >> (shift + 8)) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1);
     }
     __syncthreads();
-    if (want > 0) radix_pick(hist, want, sel);
+    radix_pick(hist, want, sel);
     __syncthreads();
   }
   const std::uint32_t K = sel[0];
   const int need = want - static_cast<int>(sel[1]);  // keys equal to K that are kept
-  std::uint32_t* keys = w.keys + blockIdx.x * kSelectMax;
-  std::int32_t* idx = w.idx + blockIdx.x * kSelectMax;
   int above_done = 0, ties_done = 0;
   for (int c0 = sl.lo; c0 < sl.hi; c0 += kSmpThreads) {
     const int i = c0 + t;
-    const bool in = want > 0 && i < sl.hi;
+    const bool in = i < sl.hi;
     const std::uint32_t key = in ? key_bits(w.p[i]) : 0u;
     const bool above = in && key > K, tie = in && key == K;
     // One exchange carries both counts: above in the high half, ties low.
@@ -619,10 +725,11 @@ __global__ void __launch_bounds__(kSmpThreads) smp_sel_local(int n, int k, SmpWo
   if (t == 0) w.part_i[blockIdx.x] = want;
 }
 
-// One workgroup: the select over every slice's candidates, each thread
-// holding a run of kRun slots in registers (vector loads, all issued at
-// once: the candidates come from other XCDs' workgroups), then the k kept,
-// ranked, into keys_sorted / idx_sorted.  With at most kSelectMax ranked
+// One workgroup: every slice's candidates, each thread holding a run of kRun
+// slots in registers (vector loads, all issued at once: the candidates come
+// from other XCDs' workgroups); up to kDirectMax of them as they are, else the
+// k that the select keeps; then the first k, ranked, into keys_sorted /
+// idx_sorted.  With at most kSelectMax ranked
 // values the rest of sampling_probabilities and sample() (sampling.cpp:36-77)
 // is short enough for one lane to run exactly as the reference does: the
 // top-p cumulative and the renormalisation sum are the same left fold over
@@ -639,11 +746,12 @@ __global__ void __launch_bounds__(kMergeThreads) smp_sel_merge(int k, float top_
   __shared__ int hist[256];
   __shared__ unsigned sel[2];
   __shared__ int wave_tot[kWaves];
-  __shared__ std::uint32_t sk[kSelectMax];
-  __shared__ std::int32_t si[kSelectMax];
+  __shared__ std::uint32_t sk[kDirectMax];
+  __shared__ std::int32_t si[kDirectMax];
+  __shared__ int rank[kDirectMax];
   __shared__ int slot;
-  if (w.st->flags & kFlagBad) return;
   const int t = threadIdx.x;
+  const int flags = w.st->flags;
   const int c_lo = t * kRun;
   // Slots past a slice's count hold stale values and are never used.
   const int valid = min(kRun, max(0, w.part_i[c_lo / kSelectMax] - c_lo % kSelectMax));
@@ -660,51 +768,83 @@ __global__ void __launch_bounds__(kMergeThreads) smp_sel_merge(int k, float top_
     sel[1] = 0u;
     slot = 0;
   }
-  for (int pass = 0; pass < 4; ++pass) {
-    const int shift = 24 - 8 * pass;
-    if (t < 256) hist[t] = 0;
-    __syncthreads();
-    const unsigned prefix = sel[0];
+  if (t < kDirectMax) rank[t] = 0;
+  __syncthreads();
+  if (flags & kFlagBad) return;
+  if (valid > 0) {
+    int q = atomicAdd(&slot, valid);
 #pragma unroll
-    for (int j = 0; j < kRun; ++j)
-      if (j < valid && (pass == 0 || (key[j] >> (shift + 8)) == prefix)) atomicAdd(&hist[(key[j] >> shift) & 255u], 1);
-    __syncthreads();
-    radix_pick(hist, k, sel);
-    __syncthreads();
-  }
-  const std::uint32_t K = sel[0];
-  const int need = k - static_cast<int>(sel[1]);
-  int my_ties = 0;
-#pragma unroll
-  for (int j = 0; j < kRun; ++j) my_ties += (j < valid && key[j] == K) ? 1 : 0;
-  int tot = 0;
-  int tie_rank = block_count_prefix<kWaves>(my_ties, wave_tot, &tot);  // the candidates are in index order
-#pragma unroll
-  for (int j = 0; j < kRun; ++j) {
-    bool keep = j < valid && key[j] > K;
-    if (j < valid && key[j] == K) keep = tie_rank++ < need;
-    if (keep) {
-      const int q = atomicAdd(&slot, 1);
-      sk[q] = key[j];
-      si[q] = id[j];
+    for (int j = 0; j < kRun; ++j) {
+      if (j < valid && q < kDirectMax) {
+        sk[q] = key[j];
+        si[q] = id[j];
+      }
+      ++q;
     }
   }
   __syncthreads();
+  int m = slot;  // candidates in sk / si
+  if (m > kDirectMax) {
+    for (int pass = 0; pass < 4; ++pass) {
+      const int shift = 24 - 8 * pass;
+      if (t < 256) hist[t] = 0;
+      __syncthreads();
+      const unsigned prefix = sel[0];
+#pragma unroll
+      for (int j = 0; j < kRun; ++j)
+        if (j < valid && (pass == 0 || (key[j] >> (shift + 8)) == prefix)) atomicAdd(&hist[(key[j] >> shift) & 255u], 1);
+      __syncthreads();
+      radix_pick(hist, k, sel);
+      __syncthreads();
+    }
+    const std::uint32_t K = sel[0];
+    const int need = k - static_cast<int>(sel[1]);
+    int my_ties = 0;
+#pragma unroll
+    for (int j = 0; j < kRun; ++j) my_ties += (j < valid && key[j] == K) ? 1 : 0;
+    int tot = 0;
+    if (t == 0) slot = 0;  // (read by every thread above, before the passes' barriers)
+    int tie_rank = block_count_prefix<kWaves>(my_ties, wave_tot, &tot);  // the candidates are in index order
+#pragma unroll
+    for (int j = 0; j < kRun; ++j) {
+      bool keep = j < valid && key[j] > K;
+      if (j < valid && key[j] == K) keep = tie_rank++ < need;
+      if (keep) {
+        const int q = atomicAdd(&slot, 1);
+        sk[q] = key[j];
+        si[q] = id[j];
+      }
+    }
+    __syncthreads();
+    m = k;
+  }
   __shared__ float rv[kSelectMax];        // the ranking's values
   __shared__ std::int32_t ri[kSelectMax]; // and indices
   __shared__ float fo[kSelectMax];        // the kept f in index order
   __shared__ std::int32_t io[kSelectMax];
   __shared__ int keep_s;
   __shared__ double s2_s;
-  if (t < k) {
-    const std::uint32_t kt = sk[t];
-    const std::int32_t it = si[t];
+  // Each candidate's rank: kDirectMax threads a quarter of the others each.
+  const int c = t % kDirectMax;
+  std::uint32_t kt = 0;
+  std::int32_t it = 0;
+  if (c < m) {
+    kt = sk[c];
+    it = si[c];
     int r = 0;
-    for (int q = 0; q < k; ++q) r += (sk[q] > kt || (sk[q] == kt && si[q] < it)) ? 1 : 0;
-    w.keys_sorted[r] = kt;
-    w.idx_sorted[r] = it;
-    rv[r] = __builtin_bit_cast(float, kt);
-    ri[r] = it;
+    for (int q = t / kDirectMax; q < m; q += kMergeThreads / kDirectMax)
+      r += (sk[q] > kt || (sk[q] == kt && si[q] < it)) ? 1 : 0;
+    if (r != 0) atomicAdd(&rank[c], r);
+  }
+  __syncthreads();
+  if (t < m) {
+    const int r = rank[t];
+    if (r < k) {
+      w.keys_sorted[r] = kt;
+      w.idx_sorted[r] = it;
+      rv[r] = __builtin_bit_cast(float, kt);
+      ri[r] = it;
+    }
   }
   __syncthreads();
   // Wave 0 runs the sequential folds with lane i holding ranked value i,
@@ -1231,13 +1371,14 @@ int smp_front(const float* logits, std::size_t n, const llmi_hip_sampling& cfg, 
   *ranked = filtering || need_ranking;
   *drawn = false;
   SmpWork& w = g_smp.w;
-  smp_max<<<kSmpBlocks, kSmpThreads, 0, s>>>(logits, ni, cfg.temperature, w, log);
-  smp_exp<<<kSmpBlocks, kSmpThreads, 0, s>>>(logits, ni, cfg.temperature, w);
+  const bool select = *ranked && k < n && k <= static_cast<std::size_t>(kSelectMax);
+  smp_max<<<kSmpBlocks, kSmpThreads, 0, s>>>(logits, ni, cfg.temperature, w);
+  smp_exp<<<kSmpBlocks, kSmpThreads, 0, s>>>(logits, ni, cfg.temperature, select ? 0 : 1, w, log);
   LLMI_TRY_HIP(hipGetLastError());
-  if (*ranked && k < n && k <= static_cast<std::size_t>(kSelectMax)) {
+  if (select) {
     // Only the first k of the ranking are read: select them.
     const int ki = static_cast<int>(k);
-    smp_sel_local<<<kSmpBlocks, kSmpThreads, 0, s>>>(ni, ki, w);
+    smp_sel_local<<<kSmpBlocks, kSmpThreads, 0, s>>>(logits, ni, cfg.temperature, ki, w);
     smp_sel_merge<<<1, kMergeThreads, 0, s>>>(ki, cfg.top_p, draw != nullptr ? draw->target : 0.0,
                                               draw != nullptr ? 1 : 0, w, draw != nullptr ? draw->also : nullptr, log);
     *drawn = draw != nullptr;
