@@ -326,7 +326,7 @@ __device__ int block_sequential_sum(F v, int m, bool has_stop, double stop_at, d
 // last workgroup of the same launch, whose atomic, barrier and second read of
 // the partials took ~3 us a kernel.  On 151,936 logits, top-k 40: smp_max 8.0 ->
 // 3.3 us, smp_exp 11.3 -> 4.3, smp_sel_local 10.4 -> 4.1 and smp_sel_merge 20 ->
-// 10.3 (with the candidate bound below), a call 66.7 -> 42.2 us.
+// 6.9 (with the candidate bound below), a call 66.7 -> 39.7 us.
 constexpr int kHeld = 8;
 
 // fn(i, src[i]) for this thread's entries of the slice; each round's loads
@@ -853,27 +853,25 @@ __global__ void __launch_bounds__(kMergeThreads) smp_sel_merge(int k, float top_
     const float v = t < k ? rv[t] : 0.0f;
     const std::int32_t vi = t < k ? ri[t] : 0;
     // sampling.cpp:36-45 and :50-53: the cumulative stops at keep - 1, where
-    // it equals the sum of the kept.
-    double cum = 0.0;
-    int keep = k;
-    bool cut = false;
+    // it equals the sum of the kept.  Lane i keeps the i-th running sum, so
+    // the additions run without a test between them (here and in the draw:
+    // the kernel went from 10.3 to 6.9 us).
+    double cum = 0.0, mine = 0.0;
 #pragma unroll
     for (int i = 0; i < kSelectMax; ++i) {
-      if (i < k && !cut) {
-        cum += static_cast<double>(readlane_f32(v, i));
-        if (top_p < 1.0f && cum >= static_cast<double>(top_p)) {
-          keep = i + 1;
-          cut = true;
-        }
-      }
+      cum += static_cast<double>(readlane_f32(v, i));
+      mine = t == i ? cum : mine;
     }
-    const double s2 = cum;
+    const unsigned long long cut =
+        __builtin_amdgcn_ballot_w64(t < k && top_p < 1.0f && mine >= static_cast<double>(top_p));
+    const int keep = cut != 0 ? __builtin_ctzll(cut) + 1 : k;
+    const double s2 = readlane_f64(mine, keep - 1);
     // The kept values renormalised, placed in index order.
-    if (t < keep) {
-      int pos = 0;
+    const std::int32_t in_order = t < keep ? vi : 0x7fffffff;
+    int pos = 0;
 #pragma unroll
-      for (int q = 0; q < kSelectMax; ++q)
-        if (q < keep) pos += __builtin_amdgcn_readlane(vi, q) < vi ? 1 : 0;
+    for (int q = 0; q < kSelectMax; ++q) pos += __builtin_amdgcn_readlane(in_order, q) < vi ? 1 : 0;
+    if (t < keep) {
       fo[pos] = renorm(v, s2);
       io[pos] = vi;
     }
@@ -892,15 +890,17 @@ __global__ void __launch_bounds__(kMergeThreads) smp_sel_merge(int k, float top_
     if (draw) {
       // sampling.cpp:66-76.  target <= 0 is reached at index 0 whatever p[0];
       // the filtered entries add +0 to the running sum.
-      id = target <= 0.0 ? 0 : -1;
-      double cum = 0.0;
+      double cum = 0.0, mine = 0.0;
 #pragma unroll
       for (int j = 0; j < kSelectMax; ++j) {
-        if (j < keep && id < 0) {
-          cum += static_cast<double>(readlane_f32(f, j));
-          if (cum >= target) id = __builtin_amdgcn_readlane(fi, j);
-        }
+        cum += static_cast<double>(readlane_f32(f, j));
+        mine = t == j ? cum : mine;
       }
+      const unsigned long long reach = __builtin_amdgcn_ballot_w64(t < keep && mine >= target);
+      if (target <= 0.0)
+        id = 0;
+      else if (reach != 0)
+        id = __builtin_amdgcn_readlane(fi, __builtin_ctzll(reach));
       // Else the last nonzero entry (never absent: the top entry's f is at
       // least 1 / keep).
       const unsigned long long nz = __builtin_amdgcn_ballot_w64(t < keep && f > 0.0f);
