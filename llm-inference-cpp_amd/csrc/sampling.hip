@@ -326,7 +326,8 @@ __device__ int block_sequential_sum(F v, int m, bool has_stop, double stop_at, d
 // last workgroup of the same launch, whose atomic, barrier and second read of
 // the partials took ~3 us a kernel.  On 151,936 logits, top-k 40: smp_max 8.0 ->
 // 3.3 us, smp_exp 11.3 -> 4.3, smp_sel_local 10.4 -> 4.1 and smp_sel_merge 20 ->
-// 6.9 (with the candidate bound below), a call 66.7 -> 39.7 us.
+// 6.9 (with the candidate bound below), a call 66.7 -> 29.6 us (the last 10 by
+// leaving out the copy of the state, see sample_device).
 constexpr int kHeld = 8;
 
 // fn(i, src[i]) for this thread's entries of the slice; each round's loads
@@ -1274,16 +1275,29 @@ struct SmpBuffers {
   unsigned* sort_below = nullptr;      // and the tiles' counts of smaller digits
   float* host_io = nullptr;  // staging for the host-pointer entry points (device)
   std::int32_t* id_dev = nullptr;
+  SampleLog* result = nullptr;  // pinned: what the kernels of a synchronous draw leave for the host
   SmpWork w{};
 };
 SmpBuffers g_smp;
 bool g_exact_only = false;
 
+}  // namespace
+
+void release_sampling_workspace() {
+  if (g_smp.base != nullptr) (void)hipFree(g_smp.base);
+  if (g_smp.result != nullptr) (void)hipHostFree(g_smp.result);
+  g_smp = SmpBuffers{};
+}
+
+namespace {
+
 int smp_reserve(std::size_t n, hipStream_t s) {
   if (n <= g_smp.cap) return LLMI_OK;
   LLMI_TRY_HIP(hipStreamSynchronize(s));
+  SampleLog* result = g_smp.result;
   if (g_smp.base != nullptr) LLMI_TRY_HIP(hipFree(g_smp.base));
   g_smp = SmpBuffers{};
+  g_smp.result = result;
   const std::size_t tiles = ceil_div(n, static_cast<std::size_t>(sort_per_tile(n)));
   auto al = [](std::size_t b) { return (b + 255) & ~static_cast<std::size_t>(255); };
   // The top-k selection writes up to kCandMax candidates into keys / idx.
@@ -1292,6 +1306,8 @@ int smp_reserve(std::size_t n, hipStream_t s) {
   const std::size_t bytes = 9 * vec + 2 * al(sizeof(unsigned) * kSortDigits * tiles) +
                             al(sizeof(double) * 2 * kSmpBlocks) + al(sizeof(int) * 2 * kSmpBlocks) +
                             al(sizeof(float) * kSmpBlocks) + al(sizeof(SmpState)) + al(sizeof(std::int32_t));
+  if (g_smp.result == nullptr)
+    LLMI_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_smp.result), sizeof(SampleLog), hipHostMallocDefault));
   LLMI_TRY_HIP(hipMalloc(&g_smp.base, bytes));
   char* c = static_cast<char*>(g_smp.base);
   auto take = [&c, &al](std::size_t b) {
@@ -1400,17 +1416,12 @@ int smp_read_state(SmpState* st, hipStream_t s) {
   return LLMI_OK;
 }
 
-int smp_bad_input(const SmpState& st) {
-  if (st.flags & kFlagNaN) return fail(LLMI_ERR_ARG, "sampling: logits / temperature has a NaN entry");
+int smp_bad_input(int flags) {
+  if (flags & kFlagNaN) return fail(LLMI_ERR_ARG, "sampling: logits / temperature has a NaN entry");
   return fail(LLMI_ERR_ARG, "sampling: logits / temperature has a +inf entry");
 }
 
 }  // namespace
-
-void release_sampling_workspace() {
-  if (g_smp.base != nullptr) (void)hipFree(g_smp.base);
-  g_smp = SmpBuffers{};
-}
 
 // Draws one index on the device; *id_host receives it.  `also` (device, may
 // be null) receives it too, on the stream, before the host learns it.
@@ -1426,19 +1437,22 @@ int sample_device(const float* logits, std::size_t n, const llmi_hip_sampling& c
     LLMI_TRY_HIP(hipStreamSynchronize(s));
     return LLMI_OK;
   }
+  // The kernels leave the index and the state in pinned memory themselves (a
+  // copy of the state by the runtime took 10 us of a 39.7 us call).
   bool ranked = false, drawn = false;
-  const FrontDraw fd{target, also, nullptr};
-  if (int rc = smp_front(logits, n, cfg, g_exact_only, s, &ranked, &drawn, &fd)) return rc;
+  SampleLog* const out = g_smp.result;
+  const FrontDraw fd{target, also, out};
+  if (int rc = smp_front(logits, n, cfg, g_exact_only, s, &ranked, &drawn, &fd, out)) return rc;
   SmpWork& w = g_smp.w;
   const int ni = static_cast<int>(n);
   if (!drawn) {
     if (g_exact_only) smp_seq_sum2<<<1, kSmpThreads, 0, s>>>(reinterpret_cast<const float*>(w.keys_sorted), w);
-    smp_draw<<<kSmpBlocks, kSmpThreads, 0, s>>>(ni, target, ranked ? 1 : 0, w, also, nullptr);
+    smp_draw<<<kSmpBlocks, kSmpThreads, 0, s>>>(ni, target, ranked ? 1 : 0, w, also, out);
   }
   LLMI_TRY_HIP(hipGetLastError());
-  SmpState st{};
-  if (int rc = smp_read_state(&st, s)) return rc;
-  if (st.flags & kFlagAllNegInf) {
+  LLMI_TRY_HIP(hipStreamSynchronize(s));
+  const int flags = out->state >> 1;
+  if (flags & kFlagAllNegInf) {
     // Every logit is -inf: the reference's probabilities are NaN and its
     // draw falls through to argmax(logits), the first entry.
     *id_host = 0;
@@ -1446,8 +1460,8 @@ int sample_device(const float* logits, std::size_t n, const llmi_hip_sampling& c
     LLMI_TRY_HIP(hipStreamSynchronize(s));
     return LLMI_OK;
   }
-  if (st.flags & kFlagBad) return smp_bad_input(st);
-  if (!st.decided) {
+  if (flags & kFlagBad) return smp_bad_input(flags);
+  if ((out->state & 1) == 0) {
     // The exact renormalisation sum, which needs the ranking.
     if (!ranked) {
       smp_keys<<<static_cast<unsigned>(ceil_div(n, kSmpThreads)), kSmpThreads, 0, s>>>(ni, w);
@@ -1455,12 +1469,12 @@ int sample_device(const float* logits, std::size_t n, const llmi_hip_sampling& c
       if (int rc = smp_sort(n, s)) return rc;
     }
     smp_seq_sum2<<<1, kSmpThreads, 0, s>>>(reinterpret_cast<const float*>(w.keys_sorted), w);
-    smp_draw<<<kSmpBlocks, kSmpThreads, 0, s>>>(ni, target, ranked ? 1 : 0, w, also, nullptr);
+    smp_draw<<<kSmpBlocks, kSmpThreads, 0, s>>>(ni, target, ranked ? 1 : 0, w, also, out);
     LLMI_TRY_HIP(hipGetLastError());
-    if (int rc = smp_read_state(&st, s)) return rc;
-    if (!st.decided) return fail(LLMI_ERR_STATE, "sampling: the exact draw did not decide (internal error)");
+    LLMI_TRY_HIP(hipStreamSynchronize(s));
+    if ((out->state & 1) == 0) return fail(LLMI_ERR_STATE, "sampling: the exact draw did not decide (internal error)");
   }
-  *id_host = st.id;
+  *id_host = out->id;
   return LLMI_OK;
 }
 
@@ -1541,7 +1555,7 @@ int llmi_hip_sampling_probabilities(const float* logits, size_t n, const llmi_hi
     for (std::size_t i = 0; i < n; ++i) probs[i] = i < k ? __builtin_nanf("") : 0.0f;
     return LLMI_OK;
   }
-  if (st.flags & kFlagBad) return smp_bad_input(st);
+  if (st.flags & kFlagBad) return smp_bad_input(st.flags);
   LLMI_TRY_HIP(hipMemcpy(probs, out, n * sizeof(float), hipMemcpyDeviceToHost));
   return LLMI_OK;
 }
