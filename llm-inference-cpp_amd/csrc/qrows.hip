@@ -466,16 +466,20 @@ void launch_form(const RowsArgs& g, const float* x, std::size_t in_, std::size_t
   // 16 rows 47.5).  From about 1.4 wavefronts per SIMD: 16 rows, blocks
   // chained in registers (896 x 896 at 512 rows 12.9, split over 8
   // wavefronts 15.1); rows of more than 32 blocks from 2.5 (at 1.75, 896 x
-  // 4864: split 60.0, not 66.2), pairs, whose split has half the wavefronts
+  // 4864: split 53.8, not 56.6), pairs, whose split has half the wavefronts
   // per group, from 0.5.  Below, split: over 8 wavefronts (4864 x 896 at 64
-  // rows 11.4, 16 wavefronts 13.6), over 16 when there are at most 256 tiles
-  // (896 x 4864 at 64 rows 13.6, 8 wavefronts 15.0).
+  // rows 10.4, 16 wavefronts 13.6), over 16 when there are at most 256 tiles
+  // (896 x 4864 at 64 rows 13.6, 8 wavefronts 15.0).  A Q8_0 wavefront of the
+  // 8 has one block in flight: the other waves cover its loads, and two cost
+  // registers (896 x 4864 at 256 and 512 rows 32.1 and 53.8, two blocks 35.9
+  // and 57.4); Q4_0's smaller blocks measure the same or better in twos (576
+  // x 1536 at 256 rows 10.2, one block 10.4).
   const std::size_t units = groups * ceil_div(rows_, 16);
   const bool pairs = FORM == kGateUp || g.mode[0] != kStorePlain;
   if (units >= 8192) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, whole, s);
   else if (units >= (pairs ? 512u : nblk <= 32 ? 1408u : 2560u)) launch_tiles<TYPE, FORM, 1>(g, x, in, nblk, rows, whole, s);
   else if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2>(g, x, in, nblk, rows, whole, s);
-  else if (units > 256) launch_split_blocks<TYPE, FORM, 1, 8, 2>(g, x, in, nblk, rows, whole, s);
+  else if (units > 256) launch_split_blocks<TYPE, FORM, 1, 8, TYPE == LLMI_TYPE_Q8_0 ? 1 : 2>(g, x, in, nblk, rows, whole, s);
   else launch_split_blocks<TYPE, FORM, 1, 16, 2>(g, x, in, nblk, rows, whole, s);
 }
 
