@@ -463,7 +463,11 @@ void launch_form(const RowsArgs& g, const float* x, std::size_t in_, std::size_t
   const std::size_t groups = static_cast<std::size_t>(g.tiles) * (FORM == kGateUp ? 8 : 4);
   // By the number of 16 x 16 tiles against the GPU's 1024 SIMDs (times in us,
   // Q8_0).  From 8192: 32 rows per wavefront (4864 x 896 at 512 rows 45.4,
-  // 16 rows 47.5).  From about 1.4 wavefronts per SIMD: 16 rows, blocks
+  // 16 rows 47.5; 151936 x 896 at 64 rows 157, 16 rows 176), unless a last
+  // half-empty 32 costs more than that saves: few 16-row groups, an odd number
+  // of them (151936 x 896 at 9 rows 80.4, 16 rows per wavefront 50.6; at 40
+  // 149, 128; 49152 x 576 at 80 50.8, 46.7; but at 176, 11 groups, 98.3,
+  // 103.0).  From about 1.4 wavefronts per SIMD: 16 rows, blocks
   // chained in registers (896 x 896 at 512 rows 12.9, split over 8
   // wavefronts 15.1); rows of more than 32 blocks from 2.5 (at 1.75, 896 x
   // 4864: split 53.8, not 56.6), pairs, whose split has half the wavefronts
@@ -474,9 +478,11 @@ void launch_form(const RowsArgs& g, const float* x, std::size_t in_, std::size_t
   // registers (896 x 4864 at 256 and 512 rows 32.1 and 53.8, two blocks 35.9
   // and 57.4); Q4_0's smaller blocks measure the same or better in twos (576
   // x 1536 at 256 rows 10.2, one block 10.4).
-  const std::size_t units = groups * ceil_div(rows_, 16);
+  const std::size_t groups16 = ceil_div(rows_, 16);
+  const std::size_t units = groups * groups16;
   const bool pairs = FORM == kGateUp || g.mode[0] != kStorePlain;
-  if (units >= 8192) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, whole, s);
+  const bool by32 = groups16 % 2 == 0 || groups16 > 8;
+  if (units >= 8192 && by32) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, whole, s);
   else if (units >= (pairs ? 512u : nblk <= 32 ? 1408u : 2560u)) launch_tiles<TYPE, FORM, 1>(g, x, in, nblk, rows, whole, s);
   else if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2>(g, x, in, nblk, rows, whole, s);
   else if (units > 256) launch_split_blocks<TYPE, FORM, 1, 8, TYPE == LLMI_TYPE_Q8_0 ? 1 : 2>(g, x, in, nblk, rows, whole, s);

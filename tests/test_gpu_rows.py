@@ -20,10 +20,11 @@ def bits(a):
 # 16-output group and a 64-row tile, of a partial block and a whole one, of
 # one block per wavefront (4, 8, 16 wavefronts) and several; 16 x 16 tiles up
 # to 256 (16 wavefronts a tile), up to 1408 / 2560 (8), up to 8191 (16 rows a
-# wavefront) and from 8192 (32 rows).
+# wavefront) and from 8192 (32 rows, but 16 for few groups of 16, an odd
+# number of them).
 SHAPES = [(9, 1, 1), (16, 15, 31), (17, 16, 32), (31, 17, 33), (32, 63, 63), (33, 65, 512), (15, 64, 513),
           (40, 130, 1055), (100, 700, 260), (48, 1500, 1024), (257, 1416, 64), (260, 1500, 1037), (529, 3900, 96),
-          (545, 3890, 35)]
+          (545, 3890, 35), (11, 131073, 33), (41, 43700, 64), (33, 43690, 35)]
 
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
