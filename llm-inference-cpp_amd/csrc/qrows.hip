@@ -142,6 +142,14 @@ __device__ __forceinline__ std::uint32_t opaque(std::uint32_t& v) {
   return v;
 }
 
+// Memory operations of the wavefront's lanes before this point come before
+// those after it; no instruction.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int kRowStride = 36;  // LDS floats per row: eight rows' 16-byte reads in distinct banks
 
 template <int TYPE, int TT, bool WHOLE>
@@ -225,13 +233,19 @@ struct RowsTile {
         for (int e = 0; e < 4; ++e) dst[u * 8 * kRowStride + e * 8] = e < left ? r.x[u][e] : 0.0f;
     }
   }
+  // The lane's operands, which other lanes of the wavefront staged.  A
+  // wavefront's LDS operations execute in order, so no wait stands around
+  // the reads, but per lane the addresses differ from the stores': the
+  // compiler is told to keep the order too.
   __device__ __forceinline__ void fragments(f32x4 (&a)[TT][2]) const {
+    wave_order();
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
       const f32x4* src = reinterpret_cast<const f32x4*>(xs + (tt * 16 + n) * kRowStride + q * 8);
       a[tt][0] = src[0];
       a[tt][1] = src[1];
     }
+    wave_order();
   }
 };
 
