@@ -852,16 +852,33 @@ int pick_chunk(int want, std::size_t rows, std::size_t nblk) {
   return 1;
 }
 
-// How a launch of `tiles` 64-row tiles runs a product of 2..8 rows on 64-row
-// tiles (GroupProblem's kinds), by measurement (us, vector ALUs / matrix
-// cores, Q4_0 and Q8_0):
+// Rows of more than 32 blocks on so few tiles that row chunks give each CU at
+// most one workgroup: the smallest such chunk on the vector ALUs, 0 if there
+// is none.  A workgroup on the matrix cores takes all the rows, which leaves
+// most CUs idle here, and the many blocks make its chain long (us, vector
+// ALUs / else): 2048 x 2048 at 3 rows 6.4 / 7.5 and, in a group, at 8 rows
+// 6.6 / 11.1; 8192 x 2560 at 4 rows 8.7 / 10.4; 144 x 1712 at 7 rows in a
+// group 7.6 / 9.4.  With 32 blocks or fewer the others are as fast (2749 x
+// 1003 at 5 rows 4.6 on 16 x 16 tiles).
+int few_chunk(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
+  constexpr std::size_t kCus = 256;
+  if (m.nblk <= 32) return 0;
+  for (int r = 1; r <= 4; r *= 2)
+    if (tiles * ceil_div(rows, r) <= kCus)
+      return r == 1 || wide_lds(m.nblk, std::min<std::size_t>(rows, r)) <= kLdsTarget ? r : 0;
+  return 0;
+}
+
+// How a launch of `tiles` 64-row tiles runs a product of 2..8 rows that
+// few_chunk has no chunk for on 64-row tiles (GroupProblem's kinds), by
+// measurement (us, vector ALUs / matrix cores, Q4_0 and Q8_0):
+//   rows of more than 64 blocks on up to 128 tiles: row chunks on several
+//     workgroups (896 x 4864 10.4 / 15.2);
 //   2 rows: the vector ALUs -- half of a 4-row matrix instruction's rows are
 //     empty -- (151936 x 896 20.4 / 24.6, 4864 x 896 4.6 / 5.0) except for
 //     Q8_0, whose codes decode for less, on many tiles (32.6 / 25.7), and for a
 //     partial last block (30000 x 700 8.0 / 5.9);
 //   3 rows of Q4_0 on many tiles: 49152 x 576 6.7 / 7.4;
-//   rows of more than 64 blocks on few tiles: row chunks on several
-//     workgroups (896 x 4864 10.4 / 15.2);
 //   else the matrix cores (151936 x 896 at 8 rows 52.3 / 33.6 and 78.2 /
 //     35.6, at 4 27.9 / 24.2 and 41.7 / 26.3).
 int few_kind(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
@@ -873,8 +890,11 @@ int few_kind(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
 
 // Wavefronts per tile on the matrix cores (4, 8 or 16; us at 8 rows, Q4_0): by
 // the tiles, enough to fill the GPU (768 tiles of 576 inputs 9.3 / 10.2 /
-// 12.5; 256 of 896 7.5 / 6.8 / 7.3; 76 7.2 / 6.3 / 5.7).
-int few_waves(std::size_t tiles) { return tiles >= 512 ? 4 : tiles >= 128 ? 8 : 16; }
+// 12.5; 256 of 896 7.5 / 6.8 / 7.3; 76 7.2 / 6.3 / 5.7); long rows keep 16
+// for longer (128 of 2560 at 5 rows 17.4 / 13.6 / 12.0).
+int few_waves(std::size_t tiles, std::size_t nblk) {
+  return tiles >= 512 ? 4 : tiles >= (nblk > 32 ? 192u : 128u) ? 8 : 16;
+}
 
 // Wavefronts per 64-row tile: each takes about kBlocksPerWave blocks (4 for
 // Q4_0, 2 for Q8_0: about 4 KB of codes and scales in flight per
@@ -915,14 +935,18 @@ TilePlan plan_single(const DeviceMatrix& m, std::size_t rows) {
     return p;
   }
   if (!wide_fits(nblk)) return p;  // rows too long for LDS staging
+  const int chunk = rows > 1 ? few_chunk(m, rows, m.ntiles) : 0;
   // Few tiles: 16-row x 16-output tiles spread the product over more CUs
   // (qrows.hip; 576 x 576 at 4 rows 3.7 us, on 64-row tiles 4.0), which
   // rows of a partial block take from two rows on (2749 x 1003 4.6, 6.8);
-  // 6 rows and more fill them better (4864 x 896 at 8 rows of Q8_0 5.9, 6.8).
-  if (rows > 1 && nblk <= 64 && m.ntiles <= (rows > 5 ? 128u : 64u) && (rows > 2 || m.in % kBlock != 0)) return p;
-  p.kind = rows == 1 ? 1 : few_kind(m, rows, m.ntiles);
+  // 6 rows and more fill them better (4864 x 896 at 8 rows of Q8_0 5.9, 6.8,
+  // but 8192 x 1800 at 6 11.4, 9.3).
+  if (rows > 1 && nblk <= 64 && m.ntiles <= (rows > 5 && nblk <= 32 ? 128u : 64u) && (rows > 2 || m.in % kBlock != 0) &&
+      chunk == 0)
+    return p;
+  p.kind = rows == 1 ? 1 : chunk != 0 ? chunk : few_kind(m, rows, m.ntiles);
   if (p.kind == GroupProblem::kFew4 || p.kind == GroupProblem::kFew8) {
-    p.waves = few_waves(m.ntiles);
+    p.waves = few_waves(m.ntiles, nblk);
     return p;
   }
   p.bpw = static_cast<int>(ceil_div(nblk, wide_waves(nblk, m.type)));
@@ -1018,8 +1042,22 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
     if (int rc = check_shape(*e.m, e.rows)) return rc;
     wide_total += e.m->ntiles * ceil_div(e.rows, 8);
   }
+  // The row chunk that few_chunk gives all of a type's products of 2..8 rows,
+  // else 0: another kind for some of them is another launch, which costs
+  // more than it saves.
+  const auto common_chunk = [&](int type) {
+    int c = -1;
+    for (std::size_t i = 0; i < count; ++i) {
+      const GroupEntry& e = entries[i];
+      if (e.rows == 1 || e.m->out == 0 || e.m->type != type) continue;
+      const int r = few_chunk(*e.m, e.rows, wide_total);
+      c = c < 0 || c == r ? r : 0;
+    }
+    return std::max(c, 0);
+  };
   // Products are launched by weight type and row chunk R (one kernel
   // instance each).
+  const int chunks[2] = {common_chunk(LLMI_TYPE_Q8_0), common_chunk(LLMI_TYPE_Q4_0)};
   for (int type : {LLMI_TYPE_Q8_0, LLMI_TYPE_Q4_0})
   for (int R : {int{GroupProblem::kNarrow}, 1, 2, 4, int{GroupProblem::kFew4}, int{GroupProblem::kFew8}}) {
     const bool few = R == GroupProblem::kFew4 || R == GroupProblem::kFew8;
@@ -1039,8 +1077,13 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
       LLMI_REQUIRE(e.prologue == kPlain || e.prologue == kRmsNorm || e.prologue == kSiluUp,
                    "group: unknown prologue");
       LLMI_REQUIRE(narrow || wide_fits(m.nblk), "group: rows too long for the grouped GEMV (in above ~10k)");
-      const int r = narrow ? int{GroupProblem::kNarrow} : e.rows == 1 ? 1 : few_kind(m, e.rows, wide_total);
-      if (r != R || m.type != type) continue;
+      if (m.type != type) continue;
+      const int chunk = chunks[type == LLMI_TYPE_Q8_0 ? 0 : 1];
+      const int r = narrow        ? int{GroupProblem::kNarrow}
+                    : e.rows == 1 ? 1
+                    : chunk != 0  ? chunk
+                                  : few_kind(m, e.rows, wide_total);
+      if (r != R) continue;
       GroupProblem p{};
       p.codes = m.codes;
       p.scales = m.scales;
@@ -1103,7 +1146,7 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
       l.lds = std::max(l.lds, need);
       plan->wg_prob.insert(plan->wg_prob.end(), wgs, static_cast<std::uint32_t>(j));
     }
-    if (few) l.waves = few_waves(wg);
+    if (few) l.waves = few_waves(wg, static_cast<std::size_t>(probs[0].nblk));
     LLMI_REQUIRE(l.lds <= max_lds_per_block(), "group: a product needs more LDS than one workgroup may use");
     l.total_wgs = static_cast<int>(wg);
     l.nprob = static_cast<int>(probs.size());

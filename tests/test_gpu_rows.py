@@ -53,9 +53,12 @@ def test_tile_edges_match_oracle(qt, rows, out, n_in):
 # 2..8 rows: one side and the other of 4 rows a matrix instruction, of a
 # 64-row tile, of a partial block; 16-row tiles (at most 64 tiles and 64
 # blocks), long rows on few tiles, and 16, 8 and 4 wavefronts per 64-row tile
-# with fewer, as many and more blocks than wavefronts.
+# with fewer, as many and more blocks than wavefronts; rows of 32 and of more
+# blocks, and those on as many row chunks of 1, 2 and 4 as there are CUs, and
+# on one more.
 FEW = [(2, 64, 33), (3, 63, 32), (4, 4161, 31), (5, 4200, 32), (8, 4097, 513), (7, 8256, 70), (4, 8192, 288),
-       (3, 32832, 100), (8, 32770, 97), (5, 32768, 160), (2, 32768, 64), (6, 200, 2100), (4, 130, 2048), (3, 8300, 2100)]
+       (3, 32832, 100), (8, 32770, 97), (5, 32768, 160), (2, 32768, 64), (6, 200, 2100), (4, 130, 2048), (3, 8300, 2100),
+       (8, 2000, 1024), (8, 2048, 1025), (8, 2049, 1056), (3, 8192, 1600), (4, 8193, 2048), (7, 8192, 1500), (5, 8193, 1030)]
 
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
@@ -81,6 +84,28 @@ def test_few_rows_match_oracle(qt, rows, out, n_in):
         got = y.download(np.float32)
         assert np.array_equal(bits(got[: rows * out]), bits(want))
         assert np.all(got[rows * out :] == 7.0)
+
+
+@pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
+@pytest.mark.parametrize("shapes", [[(8, 200, 1600), (8, 130, 2048)], [(8, 200, 1600), (8, 130, 576)],
+                                    [(8, 200, 1600), (3, 130, 1100)], [(1, 200, 1600), (8, 130, 2048)]])
+def test_groups_of_few_rows_match_oracle(qt, shapes):
+    """Products of long rows on few tiles together, with others that want
+    another kind of tile or chunk, and beside one row."""
+    orc = O.oracle()
+    keep, items, wants = [], [], []
+    for i, (rows, out, n_in) in enumerate(shapes):
+        w = synth.normal(out + 5 * n_in, out * n_in, 0.0, 0.02)
+        x = synth.normal(rows * 17 + n_in, rows * n_in, 0.0, 1.0)
+        data, scales = orc.quantize(w, out, n_in, qt)
+        wants.append(orc.matmul(x, rows, n_in, data, scales, qt, out, None))
+        xd, yd = H.DeviceBuffer.from_array(x), H.DeviceBuffer.from_array(np.full(rows * out, 7.0, dtype=np.float32))
+        keep.append((xd, yd))
+        items.append((H.Weight.upload(data, scales, out, n_in, qt), xd.ptr, yd.ptr, rows, None))
+    H.Group(items).launch()
+    H.synchronize()
+    for (_, yd), want in zip(keep, wants):
+        assert np.array_equal(bits(yd.download(np.float32)), bits(want))
 
 
 @pytest.mark.parametrize("rows", [5, 24])
