@@ -856,9 +856,9 @@ int pick_chunk(int want, std::size_t rows, std::size_t nblk) {
 // most one workgroup: the smallest such chunk on the vector ALUs, 0 if there
 // is none.  A workgroup on the matrix cores takes all the rows, which leaves
 // most CUs idle here, and the many blocks make its chain long (us, vector
-// ALUs / else): 2048 x 2048 at 3 rows 6.4 / 7.5 and, in a group, at 8 rows
-// 6.6 / 11.1; 8192 x 2560 at 4 rows 8.7 / 10.4; 144 x 1712 at 7 rows in a
-// group 7.6 / 9.4.  With 32 blocks or fewer the others are as fast (2749 x
+// ALUs / else, Q8_0): 2048 x 2048 at 3 rows 5.6 / 7.4 and, in a group, at 8
+// rows 6.1 / 11.0; 8192 x 2560 at 4 rows 9.1 / 10.9; 144 x 1712 at 7 rows in a
+// group 5.9 / 9.4.  With 32 blocks or fewer the others are as fast (2749 x
 // 1003 at 5 rows 4.6 on 16 x 16 tiles).
 int few_chunk(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
   constexpr std::size_t kCus = 256;
