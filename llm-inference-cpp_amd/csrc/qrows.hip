@@ -152,7 +152,11 @@ __device__ __forceinline__ void wave_order() {
 
 constexpr int kRowStride = 36;  // LDS floats per row: eight rows' 16-byte reads in distinct banks
 
-template <int TYPE, int TT, bool WHOLE>
+// What rows look like: whole blocks; a partial last block; of 2^25 elements
+// and more, where 32 rows are out of a 32-bit offset's reach (either).
+enum { kWhole, kRagged, kLong };
+
+template <int TYPE, int TT, int ROWS>
 struct RowsTile {
   // What a block needs from memory.
   struct Raw {
@@ -161,7 +165,7 @@ struct RowsTile {
     float sc;
   };
   const GMEM char* xb;  // the wavefront's first row (uniform)
-  using Offset = std::conditional_t<WHOLE, std::uint32_t, std::size_t>;
+  using Offset = std::conditional_t<ROWS == kLong, std::size_t, std::uint32_t>;
   Offset xo[2 * TT];  // the lane's piece of row u * 8 + lane / 8, in bytes
   const GMEM char* cb;           // the tile's codes and scales (uniform)
   const GMEM char* sb;
@@ -192,12 +196,14 @@ struct RowsTile {
     co = 16u * sub;
     so = 4u * sub;
   }
+  // FULL: block b is known to be a whole one.
+  template <bool FULL>
   __device__ __forceinline__ void load(Raw& r, int b) {
     const GMEM char* p = xb + static_cast<std::size_t>(b) * kBlock * 4;
-    if (WHOLE || b < in / kBlock) {  // (uniform) four elements at once; a row need only be 4-byte aligned
+    if (FULL || b < in / kBlock) {  // (uniform) four elements at once; a row need only be 4-byte aligned
 #pragma unroll
       for (int u = 0; u < 2 * TT; ++u) {
-        if constexpr (WHOLE) r.x[u] = *reinterpret_cast<const GMEM f32x4a4*>(p + opaque(xo[u]));
+        if constexpr (ROWS != kLong) r.x[u] = *reinterpret_cast<const GMEM f32x4a4*>(p + opaque(xo[u]));
         else r.x[u] = *reinterpret_cast<const GMEM f32x4a4*>(p + xo[u]);
       }
     } else {  // the partial block: past the row, its last element again
@@ -218,9 +224,10 @@ struct RowsTile {
   }
   // Element 4i + e of the block goes to [e][i].  Activations past `in` (the
   // last block's) become zero: the codes stored there then add nothing.
+  template <bool FULL>
   __device__ __forceinline__ void stage(const Raw& r, int b) const {
     float* dst = xs + (lane >> 3) * kRowStride + (lane & 7);
-    if (WHOLE || b < in / kBlock) {  // (uniform)
+    if (FULL || b < in / kBlock) {  // (uniform)
 #pragma unroll
       for (int u = 0; u < 2 * TT; ++u)
 #pragma unroll
@@ -256,14 +263,18 @@ struct RowsOps {
   float c[8];
   float sc;
   f32x4 part[TT];
-  __device__ __forceinline__ void products() {
+  // The sums over the block's first 4 * steps elements.
+  __device__ __forceinline__ void products(int steps) {
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) part[tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i) {
+      if (i < steps) {
 #pragma unroll
-      for (int tt = 0; tt < TT; ++tt)
-        part[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tt][i >> 2][i & 3], c[i], part[tt], 0, 0, 0);
+        for (int tt = 0; tt < TT; ++tt)
+          part[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tt][i >> 2][i & 3], c[i], part[tt], 0, 0, 0);
+      }
+    }
   }
 };
 
@@ -314,7 +325,7 @@ __device__ __forceinline__ void store_one(const RowsArgs& g, int p, int o, int r
 // registers.  A block's loads are issued before the matrix instructions of
 // the block before it; the previous block's sums are chained while the LDS
 // reads of this one's operands are under way.
-template <int TYPE, int FORM, int TT, bool WHOLE>
+template <int TYPE, int FORM, int TT, int ROWS>
 __global__ void __launch_bounds__(256, 2)
     qgemm_rows(const uint4* __restrict__ codes, const float* __restrict__ scales, const float* __restrict__ x, int in,
                int nblk, int rows, RowsArgs g) {
@@ -323,7 +334,7 @@ __global__ void __launch_bounds__(256, 2)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r0 = blockIdx.y * 16 * TT;
   const RowsPlace<FORM> at(g);
-  using Tile = RowsTile<TYPE, TT, WHOLE>;
+  using Tile = RowsTile<TYPE, TT, ROWS>;
   Tile t;
   t.init(x, in, rows, r0, lane, xs[wave]);
   at.bind(t, codes, scales, g, nblk, wave);
@@ -339,16 +350,36 @@ __global__ void __launch_bounds__(256, 2)
       for (int v = 0; v < 4; ++v) acc[tt][v] = __builtin_fmaf(o.part[tt][v], o.sc, acc[tt][v]);
   };
   typename Tile::Raw raw;
-  t.load(raw, 0);
-  for (int b = 0; b < nblk; ++b) {
-    t.stage(raw, b);
+  const auto operands = [&](int b, auto full) {
+    t.template stage<decltype(full)::value>(raw, b);
     t.fragments(o.a);
     lane_codes<TYPE>(raw.blk, t.q, o.c);
     chain();
     o.sc = raw.sc;
-    t.load(raw, min(b + 1, nblk - 1));
+  };
+  constexpr std::true_type kFull;
+  // The whole blocks but, before a partial one, the last: each loads the next
+  // (the last of a row without a partial block itself again).  The partial
+  // block's element loads stand outside the loop, and its steps past `in` are
+  // left out: 24000 x 40 Q8_0 at 424 rows 41 -> 31 us, 8192 x 1003 at 512
+  // rows (with 32-bit offsets, as whole rows have) 103 -> 87.
+  const int loop = ROWS == kWhole ? nblk : nblk - 2;
+  t.template load<ROWS == kWhole>(raw, 0);
+  for (int b = 0; b < loop; ++b) {
+    operands(b, kFull);
+    t.template load<true>(raw, ROWS == kWhole ? min(b + 1, nblk - 1) : b + 1);
     __builtin_amdgcn_sched_barrier(0);
-    o.products();
+    o.products(8);
+  }
+  if (ROWS != kWhole) {
+    if (nblk > 1) {
+      operands(nblk - 2, kFull);
+      t.template load<false>(raw, nblk - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      o.products(8);
+    }
+    operands(nblk - 1, std::false_type{});  // only its elements' steps
+    o.products((in - (nblk - 1) * kBlock + 3) / 4);
   }
   chain();
   if (!at.pairs(g)) {
@@ -385,7 +416,7 @@ __global__ void __launch_bounds__(256, 2)
 // round of KS * U blocks puts its sums and scales in LDS, and after a
 // barrier wavefront v < 4 chains accumulator register v over the round's
 // blocks in order.  G = 2: the workgroup holds both groups of a pair.
-template <int TYPE, int FORM, int G, int KS, int U, bool WHOLE>
+template <int TYPE, int FORM, int G, int KS, int U, int ROWS>
 __global__ void __launch_bounds__(64 * G * KS)
     qgemm_rows_split(const uint4* __restrict__ codes, const float* __restrict__ scales, const float* __restrict__ x,
                      int in, int nblk, int rows, RowsArgs g) {
@@ -398,26 +429,26 @@ __global__ void __launch_bounds__(64 * G * KS)
   const int half = wave / KS, kg = wave % KS;
   const int r0 = blockIdx.z * 16;
   const RowsPlace<FORM> at(g);
-  using Tile = RowsTile<TYPE, 1, WHOLE>;
+  using Tile = RowsTile<TYPE, 1, ROWS>;
   Tile t;
   t.init(x, in, rows, r0, lane, xs[wave]);
   at.bind(t, codes, scales, g, nblk, static_cast<int>(blockIdx.y) + 2 * half);
   float acc = 0.0f;
   typename Tile::Raw raw[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) t.load(raw[u], min(u * KS + kg, nblk - 1));
+  for (int u = 0; u < U; ++u) t.template load<ROWS == kWhole>(raw[u], min(u * KS + kg, nblk - 1));
   for (int b0 = 0; b0 < nblk; b0 += RB) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int b = b0 + u * KS + kg;
       if (b < nblk) {
         RowsOps<1> o;
-        t.stage(raw[u], b);
+        t.template stage<ROWS == kWhole>(raw[u], b);
         t.fragments(o.a);
         lane_codes<TYPE>(raw[u].blk, t.q, o.c);
         if (t.q == 0) ss[half][u * KS + kg][t.n] = raw[u].sc;
-        if (b + RB < nblk) t.load(raw[u], b + RB);
-        o.products();
+        if (b + RB < nblk) t.template load<ROWS == kWhole>(raw[u], b + RB);
+        o.products(8);
 #pragma unroll
         for (int v = 0; v < 4; ++v) ps[half][u * KS + kg][v][lane] = o.part[0][v];
       }
@@ -454,26 +485,29 @@ __global__ void __launch_bounds__(64 * G * KS)
 }
 
 template <int TYPE, int FORM, int TT>
-void launch_tiles(const RowsArgs& g, const float* x, int in, int nblk, int rows, bool whole, hipStream_t s) {
+void launch_tiles(const RowsArgs& g, const float* x, int in, int nblk, int rows, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(g.tiles) * (FORM == kGateUp ? 2 : 1),
                   static_cast<unsigned>(ceil_div(rows, 16 * TT)));
-  if (whole) qgemm_rows<TYPE, FORM, TT, true><<<grid, 256, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
-  else qgemm_rows<TYPE, FORM, TT, false><<<grid, 256, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
+  if (in % kBlock == 0) qgemm_rows<TYPE, FORM, TT, kWhole><<<grid, 256, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
+  else qgemm_rows<TYPE, FORM, TT, kRagged><<<grid, 256, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
 }
-template <int TYPE, int FORM, int G, int KS, int U>
-void launch_split_blocks(const RowsArgs& g, const float* x, int in, int nblk, int rows, bool whole, hipStream_t s) {
+template <int TYPE, int FORM, int G, int KS, int U, bool LONG = false>
+void launch_split_blocks(const RowsArgs& g, const float* x, int in, int nblk, int rows, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(g.tiles) * (FORM == kGateUp ? 2 : 1), 4 / G,
                   static_cast<unsigned>(ceil_div(rows, 16)));
-  if (whole) qgemm_rows_split<TYPE, FORM, G, KS, U, true><<<grid, 64 * G * KS, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
-  else qgemm_rows_split<TYPE, FORM, G, KS, U, false><<<grid, 64 * G * KS, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
+  const auto launch = [&](auto k) {
+    qgemm_rows_split<TYPE, FORM, G, KS, U, decltype(k)::value>
+        <<<grid, 64 * G * KS, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
+  };
+  if constexpr (LONG) launch(std::integral_constant<int, kLong>{});
+  else if (in % kBlock == 0) launch(std::integral_constant<int, kWhole>{});
+  else launch(std::integral_constant<int, kRagged>{});
 }
 
 template <int TYPE, int FORM>
 void launch_form(const RowsArgs& g, const float* x, std::size_t in_, std::size_t nblk_, std::size_t rows_,
                  hipStream_t s) {
   const int in = static_cast<int>(in_), nblk = static_cast<int>(nblk_), rows = static_cast<int>(rows_);
-  // Whole blocks only, and 32 rows within reach of a 32-bit offset.
-  const bool whole = in_ % kBlock == 0 && in_ < (std::size_t{1} << 25);
   const std::size_t groups = static_cast<std::size_t>(g.tiles) * (FORM == kGateUp ? 8 : 4);
   // By the number of 16 x 16 tiles against the GPU's 1024 SIMDs (times in us,
   // Q8_0).  From 8192: 32 rows per wavefront (4864 x 896 at 512 rows 45.4,
@@ -496,11 +530,16 @@ void launch_form(const RowsArgs& g, const float* x, std::size_t in_, std::size_t
   const std::size_t units = groups * groups16;
   const bool pairs = FORM == kGateUp || g.mode[0] != kStorePlain;
   const bool by32 = groups16 % 2 == 0 || groups16 > 8;
-  if (units >= 8192 && by32) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, whole, s);
-  else if (units >= (pairs ? 512u : nblk <= 32 ? 1408u : 2560u)) launch_tiles<TYPE, FORM, 1>(g, x, in, nblk, rows, whole, s);
-  else if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2>(g, x, in, nblk, rows, whole, s);
-  else if (units > 256) launch_split_blocks<TYPE, FORM, 1, 8, TYPE == LLMI_TYPE_Q8_0 ? 1 : 2>(g, x, in, nblk, rows, whole, s);
-  else launch_split_blocks<TYPE, FORM, 1, 16, 2>(g, x, in, nblk, rows, whole, s);
+  if (in_ >= (std::size_t{1} << 25)) {  // kLong: too few tiles fit memory for the others
+    if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2, true>(g, x, in, nblk, rows, s);
+    else launch_split_blocks<TYPE, FORM, 1, 16, 2, true>(g, x, in, nblk, rows, s);
+    return;
+  }
+  if (units >= 8192 && by32) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, s);
+  else if (units >= (pairs ? 512u : nblk <= 32 ? 1408u : 2560u)) launch_tiles<TYPE, FORM, 1>(g, x, in, nblk, rows, s);
+  else if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2>(g, x, in, nblk, rows, s);
+  else if (units > 256) launch_split_blocks<TYPE, FORM, 1, 8, TYPE == LLMI_TYPE_Q8_0 ? 1 : 2>(g, x, in, nblk, rows, s);
+  else launch_split_blocks<TYPE, FORM, 1, 16, 2>(g, x, in, nblk, rows, s);
 }
 
 int check_rows(const DeviceMatrix& m, std::size_t rows) {

@@ -21,10 +21,12 @@ def bits(a):
 # one block per wavefront (4, 8, 16 wavefronts) and several; 16 x 16 tiles up
 # to 256 (16 wavefronts a tile), up to 1408 / 2560 (8), up to 8191 (16 rows a
 # wavefront) and from 8192 (32 rows, but 16 for few groups of 16, an odd
-# number of them).
+# number of them); in the last two also one block, partial, and one to 31 of
+# its elements.
 SHAPES = [(9, 1, 1), (16, 15, 31), (17, 16, 32), (31, 17, 33), (32, 63, 63), (33, 65, 512), (15, 64, 513),
           (40, 130, 1055), (100, 700, 260), (48, 1500, 1024), (257, 1416, 64), (260, 1500, 1037), (529, 3900, 96),
-          (545, 3890, 35), (11, 131073, 33), (41, 43700, 64), (33, 43690, 35)]
+          (545, 3890, 35), (11, 131073, 33), (41, 43700, 64), (33, 43690, 35),
+          (545, 3890, 31), (544, 3900, 127), (545, 3890, 1), (545, 3890, 97), (48, 12000, 29), (48, 12000, 130)]
 
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
@@ -48,6 +50,20 @@ def test_tile_edges_match_oracle(qt, rows, out, n_in):
     got = yd.download(np.float32)
     assert np.array_equal(bits(got[: rows * out]), bits(want))
     assert np.all(got[rows * out :] == 7.0)
+
+
+def test_rows_past_32_bit_offsets():
+    """Rows of 2^25 elements and more: 16 of them are out of a 32-bit byte
+    offset's reach."""
+    orc = O.oracle()
+    rows, out, n_in = 11, 2, 2**25 + 37
+    rng = np.random.default_rng(25)
+    w = np.resize(rng.standard_normal(1000003, dtype=np.float32), out * n_in)
+    x = np.resize(rng.standard_normal(999983, dtype=np.float32), rows * n_in)
+    data, scales = orc.quantize(w, out, n_in, O.Q4_0)
+    got = H.Weight.upload(data, scales, out, n_in, O.Q4_0).matmul(x, rows, None)
+    want = orc.matmul(x, rows, n_in, data, scales, O.Q4_0, out, None)
+    assert np.array_equal(bits(got), bits(want))
 
 
 # 2..8 rows: one side and the other of 4 rows a matrix instruction, of a
