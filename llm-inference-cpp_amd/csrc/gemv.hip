@@ -196,11 +196,30 @@ __device__ __forceinline__ void block_sums(const GMEM uint4* __restrict__ codes,
     }
   }
   if (nfull < nblk && nfull >= b_begin && nfull < b_end) {
+    // The partial block, its loads issued together.  Lane i carries element i
+    // of each row, broadcast by v_readlane; past `in` it is +0, which leaves
+    // the chain as it is (its sums are never -0).  Loading element by element
+    // in the chain took 2 us a row (6000 x 1087 at 5 rows 13 -> 8 us).
+    const int len = in - nfull * kBlock, e = lane & (kBlock - 1);
+    const GMEM float* xt = x + nfull * kBlock + min(e, len - 1);
+    float xv[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (r < nr) xv[r] = xt[static_cast<std::size_t>(r) * in];
     const Block<TYPE> blk = load_block<TYPE, true>(codes, base + nfull, lane);
-    for (int r = 0; r < nr; ++r)
-      part[(r * nblk + nfull) * kTileRows + lane] =
-          tail_block_dot<TYPE>(blk, x + static_cast<std::size_t>(r) * in + nfull * kBlock, in - nfull * kBlock);
     scl[nfull * kTileRows + lane] = loadf<true>(scales + (base + nfull) * kTileRows + lane);
+    float c[kBlock];
+    block_codes<TYPE>(blk, c);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r < nr) {
+        const float v = e < len ? xv[r] : 0.0f;
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kBlock; ++i) sum = __builtin_fmaf(readlane_f32(v, i), c[i], sum);
+        part[(r * nblk + nfull) * kTileRows + lane] = sum;
+      }
+    }
   }
 }
 
@@ -852,20 +871,22 @@ int pick_chunk(int want, std::size_t rows, std::size_t nblk) {
   return 1;
 }
 
-// Rows of more than 32 blocks on so few tiles that row chunks give each CU at
-// most one workgroup: the smallest such chunk on the vector ALUs, 0 if there
-// is none.  A workgroup on the matrix cores takes all the rows, which leaves
-// most CUs idle here, and the many blocks make its chain long (us, vector
-// ALUs / else, Q8_0): 2048 x 2048 at 3 rows 5.6 / 7.4 and, in a group, at 8
-// rows 6.1 / 11.0; 8192 x 2560 at 4 rows 9.1 / 10.9; 144 x 1712 at 7 rows in a
-// group 5.9 / 9.4.  With 32 blocks or fewer the others are as fast (2749 x
-// 1003 at 5 rows 4.6 on 16 x 16 tiles).
-int few_chunk(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
+// Long rows on so few tiles that chunks of the input rows, two or more per
+// tile, give each CU at most one workgroup: the smallest such chunk on the
+// vector ALUs, 0 if there is none.  A workgroup on the matrix cores takes all
+// the rows, which leaves most CUs idle here, and the many blocks make its
+// chain long (us, vector ALUs / else, Q8_0): 2048 x 2048 at 3 rows 5.6 / 7.4
+// and, in a group, at 8 rows 6.1 / 11.0; 8192 x 2560 at 4 rows 9.1 / 10.9; 144
+// x 1712 at 7 rows in a group 5.9 / 9.4; 6000 x 896 at 8 rows 5.6 / 6.3.  Long
+// is more than 32 blocks, for whole blocks 32 in a group of Q4_0 and 28 of Q8_0
+// (us: 6000 x 870 at 5 rows 6.2 / 5.8; Q4_0 6000 x 896 at 6 rows in a group 6.4
+// / 6.0, alone 4096 x 896 at 8 rows 5.3 / 4.8).
+int few_chunk(const DeviceMatrix& m, std::size_t rows, std::size_t tiles, bool group) {
   constexpr std::size_t kCus = 256;
-  if (m.nblk <= 32) return 0;
-  for (int r = 1; r <= 4; r *= 2)
-    if (tiles * ceil_div(rows, r) <= kCus)
-      return r == 1 || wide_lds(m.nblk, std::min<std::size_t>(rows, r)) <= kLdsTarget ? r : 0;
+  const std::size_t lng = m.in % kBlock != 0 ? 33 : m.type == LLMI_TYPE_Q8_0 ? 28 : group ? 32 : 33;
+  if (m.nblk < lng) return 0;
+  for (std::size_t r = 1; r <= 4 && r < rows; r *= 2)
+    if (tiles * ceil_div(rows, r) <= kCus) return r == 1 || wide_lds(m.nblk, r) <= kLdsTarget ? static_cast<int>(r) : 0;
   return 0;
 }
 
@@ -877,7 +898,7 @@ int few_chunk(const DeviceMatrix& m, std::size_t rows, std::size_t tiles) {
 //   2 rows: the vector ALUs -- half of a 4-row matrix instruction's rows are
 //     empty -- (151936 x 896 20.4 / 24.6, 4864 x 896 4.6 / 5.0) except for
 //     Q8_0, whose codes decode for less, on many tiles (32.6 / 25.7), and for a
-//     partial last block (30000 x 700 8.0 / 5.9);
+//     partial last block (4864 x 870 5.1 / 4.6, 32000 x 2075 15.5 / 13.7);
 //   3 rows of Q4_0 on many tiles: 49152 x 576 6.7 / 7.4;
 //   else the matrix cores (151936 x 896 at 8 rows 52.3 / 33.6 and 78.2 /
 //     35.6, at 4 27.9 / 24.2 and 41.7 / 26.3).
@@ -935,13 +956,14 @@ TilePlan plan_single(const DeviceMatrix& m, std::size_t rows) {
     return p;
   }
   if (!wide_fits(nblk)) return p;  // rows too long for LDS staging
-  const int chunk = rows > 1 ? few_chunk(m, rows, m.ntiles) : 0;
+  const int chunk = rows > 1 ? few_chunk(m, rows, m.ntiles, false) : 0;
   // Few tiles: 16-row x 16-output tiles spread the product over more CUs
   // (qrows.hip; 576 x 576 at 4 rows 3.7 us, on 64-row tiles 4.0), which
   // rows of a partial block take from two rows on (2749 x 1003 4.6, 6.8);
-  // 6 rows and more fill them better (4864 x 896 at 8 rows of Q8_0 5.9, 6.8,
-  // but 8192 x 1800 at 6 11.4, 9.3).
-  if (rows > 1 && nblk <= 64 && m.ntiles <= (rows > 5 && nblk <= 32 ? 128u : 64u) && (rows > 2 || m.in % kBlock != 0) &&
+  // 6 rows and more fill them better (4864 x 896 at 8 rows of Q8_0 5.9, 6.8;
+  // 6000 x 2048 10.3, 11.0, but 8192 x 1800 at 6 11.4, 9.3).
+  const std::size_t few_tiles = rows <= 5 ? 64 : nblk <= 32 ? 128 : 96;
+  if (rows > 1 && nblk <= 64 && m.ntiles <= few_tiles && (rows > 2 || m.in % kBlock != 0) &&
       chunk == 0)
     return p;
   p.kind = rows == 1 ? 1 : chunk != 0 ? chunk : few_kind(m, rows, m.ntiles);
@@ -1050,7 +1072,7 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
     for (std::size_t i = 0; i < count; ++i) {
       const GroupEntry& e = entries[i];
       if (e.rows == 1 || e.m->out == 0 || e.m->type != type) continue;
-      const int r = few_chunk(*e.m, e.rows, wide_total);
+      const int r = few_chunk(*e.m, e.rows, wide_total, true);
       c = c < 0 || c == r ? r : 0;
     }
     return std::max(c, 0);

@@ -124,19 +124,20 @@ def test_groups_of_few_rows_match_oracle(qt, shapes):
         assert np.array_equal(bits(yd.download(np.float32)), bits(want))
 
 
-@pytest.mark.parametrize("rows", [5, 24])
+@pytest.mark.parametrize("rows,out,n_in", [(5, 4500, 96), (24, 4500, 96), (5, 200, 1101), (8, 5000, 1119), (24, 4500, 65)])
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
-def test_extreme_rows_stay_in_their_rows(qt, rows):
-    """Subnormal, zero, huge and infinite activations: each row's results are
-    the oracle's, whatever its neighbours in the tile hold."""
+def test_extreme_rows_stay_in_their_rows(qt, rows, out, n_in):
+    """Subnormal, zero, huge and infinite activations, also in a partial last
+    block: each row's results are the oracle's, whatever its neighbours in the
+    tile hold."""
     orc = O.oracle()
-    out, n_in = 4500, 96
     w = synth.normal(1, out * n_in, 0.0, 0.02)
     x = synth.normal(2, rows * n_in, 0.0, 1.0).reshape(rows, n_in)
     x[0] *= np.float32(1e-42)
     x[1] = -0.0
     x[2] *= np.float32(1e36)
     x[3, 7] = np.inf
+    x[4, n_in - 1] = -np.inf
     data, scales = orc.quantize(w, out, n_in, qt)
     scales[::7] *= np.float32(1e-12)
     dev = H.Weight.upload(data, scales, out, n_in, qt)
