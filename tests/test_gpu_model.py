@@ -385,6 +385,35 @@ def test_prefill_attention_matches_reference(hidden, heads, kv):
     cm.close()
 
 
+@pytest.mark.parametrize("qt", [H.Q8_0, H.Q4_0])
+@pytest.mark.parametrize("hidden,heads", [(2048, 32), (400, 5)])
+def test_long_prompt_on_many_tiles_matches_reference(qt, hidden, heads):
+    """A prompt long enough for 32 rows per wavefront (8192 16 x 16 tiles and
+    more) in gate/up, whose output is ragged and, at 400, whose input ends in
+    a partial block, and at 2048 (head size 64) also in the q/k/v launch, with
+    RoPE and the cache writes; after prompts that take them split over
+    wavefronts and with 16 rows per wavefront; with a last group of rows that
+    is not full.  Every position's logits equal the reference's bit for
+    bit."""
+    cpu = O.reference() or O.oracle()
+    cfg = dict(arch=1, vocab_size=64, hidden_size=hidden, intermediate_size=3000, num_layers=1, num_heads=heads,
+               num_kv_heads=heads, max_position_embeddings=512, rms_norm_eps=1e-6, rope_theta=10000.0,
+               tie_word_embeddings=1, qkv_bias=1)
+    tensors = synth.make_tensors(cfg, hidden + qt, "bench")
+    gm = H.Model(cfg, tensors, qt)
+    cm = O.CpuModel(cpu, cfg, tensors, qt)
+    ids = synth.uniform_ids(hidden + 7, 405, cfg["vocab_size"])
+    cache = gm.new_cache(405)
+    assert cm.new_cache(405)
+    for a, b in ((0, 15), (15, 60), (60, 405)):
+        got = gm.forward_cached(cache, ids[a:b], all_positions=True)
+        want = cm.forward_cached(ids[a:b], all_positions=True)
+        assert np.array_equal(bits(got), bits(want)), (hidden, qt, a, b)
+    cache.free()
+    gm.free()
+    cm.close()
+
+
 def test_prefill_attention_past_the_lds_scores():
     """The workgroup-per-tile kernel holds a 16-row tile's scores in LDS up to
     about 1850 positions: a first chunk of 1200 positions takes it, a second
