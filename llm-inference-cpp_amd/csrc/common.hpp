@@ -267,7 +267,8 @@ int launch_dequantize_rows(const DeviceMatrix& m, const std::int32_t* ids, std::
 int launch_matmul(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, hipStream_t s,
                   bool accumulate = false);
 // launch_matmul's product for quantized weights and any number of rows, on
-// the matrix cores (qrows.hip); launch_matmul takes it above 8 rows.
+// the matrix cores (qrows.hip); launch_matmul takes it above 8 rows, and for
+// 2..8 where their 64-row tiles are few or their rows too long for those.
 int launch_rows(const DeviceMatrix& m, const float* x, std::size_t rows, const float* bias, float* y, hipStream_t s,
                 bool accumulate);
 // Products of one weight type and input size sharing x and rows (the

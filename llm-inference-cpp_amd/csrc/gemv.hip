@@ -14,7 +14,7 @@
 // broadcast to the fused multiply-adds.  Every code byte and scale is read
 // from HBM once; the kernels are HBM-bound at batch 1.
 //
-// qgemv_tile (batch 1; 2 and 3 rows and long rows by few_kind): one workgroup
+// qgemv_tile (batch 1; 2..8 rows by few_chunk and few_kind): one workgroup
 // per (64-row tile, chunk of up to R input rows).  Its W wavefronts split the
 // tile's blocks into contiguous ranges; each decodes a block once and forms
 // the block sums of every input row of the chunk, which it parks in LDS

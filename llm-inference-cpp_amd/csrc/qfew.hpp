@@ -12,9 +12,12 @@
 // registers feed the 32 steps of a block, and a row's 32 activations are one
 // coalesced 128-byte load.
 //
-// Bound: HBM for the weights at 4 rows; at 8 rows the fp32 units (per block
-// of 64 outputs 64 matrix instructions of 4.2 ns and, for Q4_0, 60 decoding
-// instructions of 1.2 to 1.9).  The W wavefronts take a tile's blocks in
+// Bound: HBM for the weights at 4 rows; at 8 rows the fp32 units, in part (per
+// block of 64 outputs 64 matrix instructions of 4.2 ns and, for Q4_0, 60
+// decoding instructions of 1.2 to 1.9: 17 and 5 to 7 of the 33.6 us of
+// SmolLM2's 211 products; the other 10 are the barrier, the LDS exchange and
+// the loads -- of the wavefronts' time 60 % waits to issue and 28 % at a wait
+// or barrier).  The W wavefronts take a tile's blocks in
 // turn, one per iteration, loaded kAhead iterations earlier; an iteration's
 // block sums and scales meet in one of two LDS buffers, and after its
 // barrier wavefront w advances the chains of rows w, w + W, ... over the W
@@ -22,8 +25,8 @@
 // wavefronts share a SIMD, so one workgroup's barriers run under another's
 // arithmetic, and rows of any length take 8 input rows per pass over the
 // weights.  Measured, before on the vector ALUs -> here: 151936 x 896 at 8
-// rows Q8_0 78.2 -> 35.6 us (4.6 TB/s), Q4_0 51.9 -> 32.6; SmolLM2's 211
-// products at batch 8 in one launch, Q4_0, 81.9 -> 35.4 us (decoding a word's
+// rows Q8_0 78.2 -> 36.7 us (4.3 TB/s), Q4_0 51.9 -> 33.5; SmolLM2's 211
+// products at batch 8 in one launch, Q4_0, 81.9 -> 33.6 us (decoding a word's
 // codes apart from its matrix instructions, to save their wait states, 41.1;
 // a whole row's sums in LDS, as batch 1 keeps them, 46.9).
 #pragma once

@@ -26,12 +26,15 @@
 // offsets, four multiply-adds per 16 x 16 block sums for the chain.  A
 // layout that put the workgroup's activations through LDS behind a barrier
 // per step ran at half the speed: 0.27 us per barrier, and 20 of 60 us in
-// moves and address arithmetic.
+// moves and address arithmetic.  LDS is the other part of the bound: each
+// wavefront stages its own copy of the rows, and with the bank conflicts of
+// kRowStride a CU's LDS is busy for about half of the 47 us of 512 rows of
+// 4864 x 896, whose matrix instructions take 28.7.
 //
 // Measured (Q8_0, before on VALU chains -> here): 512 rows of 4864 x 896
-// 88.3 -> 45.2 us (99 TFLOP/s), of 896 x 4864 143 -> 60.0, of 896 x 896
-// 21.8 -> 12.3; 128 rows of 576 x 576 6.1 -> 4.9; 9 rows of 896 x 4864 14.7
-// -> 12.6; one Qwen2.5 layer's seven products at 512 rows 407 -> 189.
+// 88.3 -> 46.9 us (95 TFLOP/s), of 896 x 4864 143 -> 56.6, of 896 x 896
+// 21.8 -> 11.9; 128 rows of 576 x 576 6.1 -> 5.3; 9 rows of 896 x 4864 14.7
+// -> 13.1; one Qwen2.5 layer's seven products at 512 rows 407 -> 175.
 #include <type_traits>
 
 #include "common.hpp"
@@ -129,11 +132,6 @@ __device__ __forceinline__ void lane_codes(const Block<TYPE>& b, int q, float* c
   }
 }
 
-// One wavefront's share of a product: TT groups of 16 rows x 16 outputs, one
-// block of 32 elements at a time.  Its loads, its LDS rows and its matrix
-// instructions need no other wavefront, so no barrier stands between the
-// blocks.  Addresses are a wavefront-uniform base, advanced by scalar
-// arithmetic, plus a constant offset per lane.
 // A 32-bit lane offset that stays one: widened inside the loop (by the load's
 // own addressing mode) instead of once before it, where it would cost a
 // 64-bit vector addition per load.
@@ -150,12 +148,20 @@ __device__ __forceinline__ void wave_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int kRowStride = 36;  // LDS floats per row: eight rows' 16-byte reads in distinct banks
+// LDS floats per row: rows start on 16 bytes, eight rows' reads in distinct
+// banks; of a store's eight rows the first and the last share four.  Counted:
+// 4.0 conflict cycles per LDS instruction, reads and stores together.
+constexpr int kRowStride = 36;
 
 // What rows look like: whole blocks; a partial last block; of 2^25 elements
 // and more, where 32 rows are out of a 32-bit offset's reach (either).
 enum { kWhole, kRagged, kLong };
 
+// One wavefront's share of a product: TT groups of 16 rows x 16 outputs, one
+// block of 32 elements at a time.  Its loads, its LDS rows and its matrix
+// instructions need no other wavefront, so no barrier stands between the
+// blocks.  Addresses are a wavefront-uniform base, advanced by scalar
+// arithmetic, plus a constant offset per lane.
 template <int TYPE, int TT, int ROWS>
 struct RowsTile {
   // What a block needs from memory.
