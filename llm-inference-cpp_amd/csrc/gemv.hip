@@ -1015,6 +1015,48 @@ void launch_typed(const DeviceMatrix& m, const float* x, std::size_t rows, const
   }
 }
 
+// The kinds of a group's products on 64-row tiles (`total` of them in all).
+// Products of different kinds are different launches, one after another, so
+// products of one type agree where they can, the heaviest deciding (us, one
+// kind each / agreed, Q4_0: 2048 x 2048, 500 x 1024 and 300 x 700 at 2 rows
+// 11.0 / 6.9).  Rows of more than 64 blocks go by themselves: few of them, as
+// a layer's down projection, would keep a launch of short ones waiting for
+// their chains (a Qwen2.5 layer's seven products in one launch / by
+// themselves: Q4_0 at 5 rows 24.1 / 17.6, Q8_0 24.3 / 19.8, but at 4 rows of
+// Q8_0 17.6 / 18.7).
+std::vector<int> group_kinds(const GroupEntry* entries, std::size_t count, std::size_t total) {
+  constexpr std::size_t kLong = 64;
+  std::vector<int> kinds(count, 1);
+  for (int type : {LLMI_TYPE_Q8_0, LLMI_TYPE_Q4_0})
+  for (bool lng : {false, true}) {
+    std::vector<std::size_t> of;
+    std::size_t tiles = 0, heaviest = 0;
+    for (std::size_t i = 0; i < count; ++i) {
+      const DeviceMatrix& m = *entries[i].m;
+      if (entries[i].rows == 1 || m.out == 0 || m.type != type || (m.nblk > kLong) != lng) continue;
+      if (of.empty() || m.code_bytes > entries[heaviest].m->code_bytes) heaviest = i;
+      of.push_back(i);
+      tiles += m.ntiles;
+    }
+    bool chunked = true;  // few_chunk has the same chunk for all
+    for (std::size_t i : of) {
+      kinds[i] = few_chunk(*entries[i].m, entries[i].rows, tiles, true);
+      chunked = chunked && kinds[i] != 0 && kinds[i] == kinds[of[0]];
+    }
+    if (chunked) continue;
+    for (std::size_t i : of) kinds[i] = few_kind(*entries[i].m, entries[i].rows, lng ? tiles : total);
+    if (of.empty()) continue;
+    const int k = kinds[heaviest];
+    const auto on_cores = [](int kind) { return kind == GroupProblem::kFew4 || kind == GroupProblem::kFew8; };
+    for (std::size_t i : of) {
+      const GroupEntry& e = entries[i];
+      if (on_cores(k)) kinds[i] = e.rows <= 4 ? GroupProblem::kFew4 : GroupProblem::kFew8;
+      else if (on_cores(kinds[i]) && pick_chunk(k, e.rows, e.m->nblk) == k) kinds[i] = k;
+    }
+  }
+  return kinds;
+}
+
 int check_shape(const DeviceMatrix& m, std::size_t rows) {
   LLMI_REQUIRE(m.in > 0, "matmul: in must be positive");
   LLMI_REQUIRE(m.in <= 0x7FFFFFFFu && m.out <= 0x7FFFFFFFu, "matmul: shape too large");
@@ -1064,22 +1106,9 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
     if (int rc = check_shape(*e.m, e.rows)) return rc;
     wide_total += e.m->ntiles * ceil_div(e.rows, 8);
   }
-  // The row chunk that few_chunk gives all of a type's products of 2..8 rows,
-  // else 0: another kind for some of them is another launch, which costs
-  // more than it saves.
-  const auto common_chunk = [&](int type) {
-    int c = -1;
-    for (std::size_t i = 0; i < count; ++i) {
-      const GroupEntry& e = entries[i];
-      if (e.rows == 1 || e.m->out == 0 || e.m->type != type) continue;
-      const int r = few_chunk(*e.m, e.rows, wide_total, true);
-      c = c < 0 || c == r ? r : 0;
-    }
-    return std::max(c, 0);
-  };
   // Products are launched by weight type and row chunk R (one kernel
   // instance each).
-  const int chunks[2] = {common_chunk(LLMI_TYPE_Q8_0), common_chunk(LLMI_TYPE_Q4_0)};
+  const std::vector<int> kinds = group_kinds(entries, count, wide_total);
   for (int type : {LLMI_TYPE_Q8_0, LLMI_TYPE_Q4_0})
   for (int R : {int{GroupProblem::kNarrow}, 1, 2, 4, int{GroupProblem::kFew4}, int{GroupProblem::kFew8}}) {
     const bool few = R == GroupProblem::kFew4 || R == GroupProblem::kFew8;
@@ -1100,11 +1129,7 @@ int plan_group(const GroupEntry* entries, std::size_t count, GroupPlan* plan) {
                    "group: unknown prologue");
       LLMI_REQUIRE(narrow || wide_fits(m.nblk), "group: rows too long for the grouped GEMV (in above ~10k)");
       if (m.type != type) continue;
-      const int chunk = chunks[type == LLMI_TYPE_Q8_0 ? 0 : 1];
-      const int r = narrow        ? int{GroupProblem::kNarrow}
-                    : e.rows == 1 ? 1
-                    : chunk != 0  ? chunk
-                                  : few_kind(m, e.rows, wide_total);
+      const int r = narrow ? int{GroupProblem::kNarrow} : kinds[i];
       if (r != R) continue;
       GroupProblem p{};
       p.codes = m.codes;

@@ -104,13 +104,16 @@ def test_few_rows_match_oracle(qt, rows, out, n_in):
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
 @pytest.mark.parametrize("shapes", [[(8, 200, 1600), (8, 130, 2048)], [(8, 200, 1600), (8, 130, 576)],
-                                    [(8, 200, 1600), (3, 130, 1100)], [(1, 200, 1600), (8, 130, 2048)]])
+                                    [(8, 200, 1600), (3, 130, 1100)], [(1, 200, 1600), (8, 130, 2048)],
+                                    [(2, 2000, 2048), (2, 130, 1000), (3, 70, 700)], [(2, 100, 96), (2, 3000, 700), (7, 60, 64)],
+                                    [(5, 700, 576), (5, 130, 2100), (8, 100, 3000), (1, 64, 4100)]])
 def test_groups_of_few_rows_match_oracle(qt, shapes):
     """Products of long rows on few tiles together, with others that want
-    another kind of tile or chunk, and beside one row."""
+    another kind of tile or chunk, and beside one row; the same of the other
+    type in the same group."""
     orc = O.oracle()
     keep, items, wants = [], [], []
-    for i, (rows, out, n_in) in enumerate(shapes):
+    for qt, (rows, out, n_in) in [(t, sh) for sh in shapes for t in (qt, O.Q8_0 + O.Q4_0 - qt)]:
         w = synth.normal(out + 5 * n_in, out * n_in, 0.0, 0.02)
         x = synth.normal(rows * 17 + n_in, rows * n_in, 0.0, 1.0)
         data, scales = orc.quantize(w, out, n_in, qt)
