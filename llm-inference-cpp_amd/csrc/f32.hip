@@ -185,8 +185,9 @@ int launch_matmul_f32(const DeviceMatrix& m, const float* x, std::size_t rows, c
   // has.  The line lies where the two met (us, dots / matrix cores): 896 x 896
   // at 32 rows 7.7 / 8.3, at 64 12.9 / 8.4; 576 x 576 at 64 7.0 / 6.4; 4864 x
   // 896 at 8 10.5 / 8.8; 896 x 4864 at 32 34.9 / 33.7; 49152 x 576 at 2 rows
-  // 30.9 / 18.9.
-  if (m.in >= 16 && rows > 1 && rows * m.out >= 24000 + 5600000 / m.in) {
+  // 30.9 / 18.9; not below the 24576 dots that give every CU six workgroups:
+  // 2048 x 12000 at 12 rows 68.9 / 94.4.
+  if (m.in >= 16 && rows > 1 && rows * m.out > 24600 + 5600000 / m.in) {
     if (rows <= 16) {
       const dim3 grid(static_cast<unsigned>(ceil_div(m.out, 64)), 1);
       matmul_f32_rows<1><<<grid, 256, 0, s>>>(x, w, bias, y, in, out, nr, accumulate ? 1 : 0);
