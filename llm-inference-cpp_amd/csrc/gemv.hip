@@ -141,6 +141,19 @@ __device__ __noinline__ float tail_block_dot(const Block<TYPE> blk, XP __restric
   return part;
 }
 
+// Block sum of a block whose activation i is in lane i of v.  Not inlined, so
+// that the partial block costs the loop over the whole ones no registers
+// (SmolLM2's 211 Q4_0 products at batch 1 17.21 us inlined, 17.04 so).
+template <int TYPE>
+__device__ __noinline__ float lanes_dot(const Block<TYPE> blk, float v) {
+  float c[kBlock];
+  block_codes<TYPE>(blk, c);
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kBlock; ++i) sum = __builtin_fmaf(readlane_f32(v, i), c[i], sum);
+  return sum;
+}
+
 // Block sums of blocks [b_begin, b_end) of one tile for input rows [0, nr)
 // (nr <= R; row r starts at x + r*in) into part[(r*nblk + b)*64 + lane], and
 // the blocks' scales into scl[b*64 + lane].  Loads run CH blocks ahead.
@@ -208,18 +221,9 @@ __device__ __forceinline__ void block_sums(const GMEM uint4* __restrict__ codes,
       if (r < nr) xv[r] = xt[static_cast<std::size_t>(r) * in];
     const Block<TYPE> blk = load_block<TYPE, true>(codes, base + nfull, lane);
     scl[nfull * kTileRows + lane] = loadf<true>(scales + (base + nfull) * kTileRows + lane);
-    float c[kBlock];
-    block_codes<TYPE>(blk, c);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (r < nr) {
-        const float v = e < len ? xv[r] : 0.0f;
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < kBlock; ++i) sum = __builtin_fmaf(readlane_f32(v, i), c[i], sum);
-        part[(r * nblk + nfull) * kTileRows + lane] = sum;
-      }
-    }
+    for (int r = 0; r < R; ++r)
+      if (r < nr) part[(r * nblk + nfull) * kTileRows + lane] = lanes_dot<TYPE>(blk, e < len ? xv[r] : 0.0f);
   }
 }
 
@@ -878,12 +882,13 @@ int pick_chunk(int want, std::size_t rows, std::size_t nblk) {
 // chain long (us, vector ALUs / else, Q8_0): 2048 x 2048 at 3 rows 5.6 / 7.4
 // and, in a group, at 8 rows 6.1 / 11.0; 8192 x 2560 at 4 rows 9.1 / 10.9; 144
 // x 1712 at 7 rows in a group 5.9 / 9.4; 6000 x 896 at 8 rows 5.6 / 6.3.  Long
-// is more than 32 blocks, for whole blocks 32 in a group of Q4_0 and 28 of Q8_0
-// (us: 6000 x 870 at 5 rows 6.2 / 5.8; Q4_0 6000 x 896 at 6 rows in a group 6.4
-// / 6.0, alone 4096 x 896 at 8 rows 5.3 / 4.8).
+// is 33 whole blocks, from 3 rows on 32 in a group of Q4_0 and 28 of Q8_0, and
+// 41 with a partial one (us: Q4_0 6000 x 1100 at 5 rows 7.6 / 7.2, 6000 x 896
+// at 6 rows in a group 6.4 / 6.0, alone 4096 x 896 at 8 rows 5.3 / 4.8; Q8_0
+// 2000 x 896 at 2 rows 4.6 / 4.3).
 int few_chunk(const DeviceMatrix& m, std::size_t rows, std::size_t tiles, bool group) {
   constexpr std::size_t kCus = 256;
-  const std::size_t lng = m.in % kBlock != 0 ? 33 : m.type == LLMI_TYPE_Q8_0 ? 28 : group ? 32 : 33;
+  const std::size_t lng = m.in % kBlock != 0 ? 41 : rows == 2 ? 33 : m.type == LLMI_TYPE_Q8_0 ? 28 : group ? 32 : 33;
   if (m.nblk < lng) return 0;
   for (std::size_t r = 1; r <= 4 && r < rows; r *= 2)
     if (tiles * ceil_div(rows, r) <= kCus) return r == 1 || wide_lds(m.nblk, r) <= kLdsTarget ? static_cast<int>(r) : 0;

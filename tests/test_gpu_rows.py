@@ -74,7 +74,8 @@ def test_rows_past_32_bit_offsets():
 # on one more.
 FEW = [(2, 64, 33), (3, 63, 32), (4, 4161, 31), (5, 4200, 32), (8, 4097, 513), (7, 8256, 70), (4, 8192, 288),
        (3, 32832, 100), (8, 32770, 97), (5, 32768, 160), (2, 32768, 64), (6, 200, 2100), (4, 130, 2048), (3, 8300, 2100),
-       (8, 2000, 1024), (8, 2048, 1025), (8, 2049, 1056), (3, 8192, 1600), (4, 8193, 2048), (7, 8192, 1500), (5, 8193, 1030)]
+       (8, 2000, 1024), (8, 2048, 1025), (8, 2049, 1056), (3, 8192, 1600), (4, 8193, 2048), (7, 8192, 1500), (5, 8193, 1030),
+       (8, 2000, 1279), (8, 2000, 1281), (5, 4100, 1290)]
 
 
 @pytest.mark.parametrize("qt", [O.Q8_0, O.Q4_0])
