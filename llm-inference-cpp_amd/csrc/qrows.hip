@@ -153,9 +153,10 @@ __device__ __forceinline__ void wave_order() {
 // 4.0 conflict cycles per LDS instruction, reads and stores together.
 constexpr int kRowStride = 36;
 
-// What rows look like: whole blocks; a partial last block; of 2^25 elements
-// and more, where 32 rows are out of a 32-bit offset's reach (either).
+// What rows look like: whole blocks; a partial last block; either, with 64-bit
+// offsets: from kLongFrom elements 32 rows are out of a 32-bit one's reach.
 enum { kWhole, kRagged, kLong };
+constexpr int kLongFrom = 1 << 25;
 
 // One wavefront's share of a product: TT groups of 16 rows x 16 outputs, one
 // block of 32 elements at a time.  Its loads, its LDS rows and its matrix
@@ -202,6 +203,11 @@ struct RowsTile {
     co = 16u * sub;
     so = 4u * sub;
   }
+  // Where the reads are ordered before the next block's stores: after them,
+  // which keeps the next loads below them too, or before the stores (us at 512
+  // rows, after / before: Q8_0 896 x 896 12.1 / 13.0, 4864 x 896 44.7 / 45.6,
+  // Q4_0 4864 x 896 45.1 / 45.7, but 2048 x 4864 105.3 / 102.2).
+  static constexpr bool kOrderAfterReads = TYPE == LLMI_TYPE_Q8_0 || TT == 2;
   // FULL: block b is known to be a whole one.
   template <bool FULL>
   __device__ __forceinline__ void load(Raw& r, int b) {
@@ -232,6 +238,7 @@ struct RowsTile {
   // last block's) become zero: the codes stored there then add nothing.
   template <bool FULL>
   __device__ __forceinline__ void stage(const Raw& r, int b) const {
+    if (!kOrderAfterReads) wave_order();
     float* dst = xs + (lane >> 3) * kRowStride + (lane & 7);
     if (FULL || b < in / kBlock) {  // (uniform)
 #pragma unroll
@@ -258,7 +265,7 @@ struct RowsTile {
       a[tt][0] = src[0];
       a[tt][1] = src[1];
     }
-    wave_order();
+    if (kOrderAfterReads) wave_order();
   }
 };
 
@@ -368,7 +375,7 @@ __global__ void __launch_bounds__(256, 2)
   // (the last of a row without a partial block itself again).  The partial
   // block's element loads stand outside the loop, and its steps past `in` are
   // left out: 24000 x 40 Q8_0 at 424 rows 41 -> 31 us, 8192 x 1003 at 512
-  // rows (with 32-bit offsets, as whole rows have) 103 -> 87.
+  // rows (with 32-bit offsets, as whole rows have) 103 -> 83.
   const int loop = ROWS == kWhole ? nblk : nblk - 2;
   t.template load<ROWS == kWhole>(raw, 0);
   for (int b = 0; b < loop; ++b) {
@@ -497,17 +504,16 @@ void launch_tiles(const RowsArgs& g, const float* x, int in, int nblk, int rows,
   if (in % kBlock == 0) qgemm_rows<TYPE, FORM, TT, kWhole><<<grid, 256, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
   else qgemm_rows<TYPE, FORM, TT, kRagged><<<grid, 256, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
 }
-template <int TYPE, int FORM, int G, int KS, int U, bool LONG = false>
+// 32-bit offsets measure 2 to 6 % slower in the split form of ragged rows
+// (320 x 1003 of Q4_0 at 1000 rows 14.9 us against 14.0), so it takes kLong's.
+template <int TYPE, int FORM, int G, int KS, int U>
 void launch_split_blocks(const RowsArgs& g, const float* x, int in, int nblk, int rows, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(g.tiles) * (FORM == kGateUp ? 2 : 1), 4 / G,
                   static_cast<unsigned>(ceil_div(rows, 16)));
-  const auto launch = [&](auto k) {
-    qgemm_rows_split<TYPE, FORM, G, KS, U, decltype(k)::value>
-        <<<grid, 64 * G * KS, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
-  };
-  if constexpr (LONG) launch(std::integral_constant<int, kLong>{});
-  else if (in % kBlock == 0) launch(std::integral_constant<int, kWhole>{});
-  else launch(std::integral_constant<int, kRagged>{});
+  if (in % kBlock == 0 && in < kLongFrom)
+    qgemm_rows_split<TYPE, FORM, G, KS, U, kWhole><<<grid, 64 * G * KS, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
+  else
+    qgemm_rows_split<TYPE, FORM, G, KS, U, kLong><<<grid, 64 * G * KS, 0, s>>>(g.codes[0], g.scales[0], x, in, nblk, rows, g);
 }
 
 template <int TYPE, int FORM>
@@ -536,13 +542,9 @@ void launch_form(const RowsArgs& g, const float* x, std::size_t in_, std::size_t
   const std::size_t units = groups * groups16;
   const bool pairs = FORM == kGateUp || g.mode[0] != kStorePlain;
   const bool by32 = groups16 % 2 == 0 || groups16 > 8;
-  if (in_ >= (std::size_t{1} << 25)) {  // kLong: too few tiles fit memory for the others
-    if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2, true>(g, x, in, nblk, rows, s);
-    else launch_split_blocks<TYPE, FORM, 1, 16, 2, true>(g, x, in, nblk, rows, s);
-    return;
-  }
-  if (units >= 8192 && by32) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, s);
-  else if (units >= (pairs ? 512u : nblk <= 32 ? 1408u : 2560u)) launch_tiles<TYPE, FORM, 1>(g, x, in, nblk, rows, s);
+  const bool split = in >= kLongFrom;  // too few tiles fit memory for the others
+  if (units >= 8192 && by32 && !split) launch_tiles<TYPE, FORM, 2>(g, x, in, nblk, rows, s);
+  else if (units >= (pairs ? 512u : nblk <= 32 ? 1408u : 2560u) && !split) launch_tiles<TYPE, FORM, 1>(g, x, in, nblk, rows, s);
   else if (pairs) launch_split_blocks<TYPE, FORM, 2, 4, 2>(g, x, in, nblk, rows, s);
   else if (units > 256) launch_split_blocks<TYPE, FORM, 1, 8, TYPE == LLMI_TYPE_Q8_0 ? 1 : 2>(g, x, in, nblk, rows, s);
   else launch_split_blocks<TYPE, FORM, 1, 16, 2>(g, x, in, nblk, rows, s);

@@ -40,15 +40,22 @@ def kernels(tmp_path_factory):
 
 
 def test_lds_staging_is_ordered(kernels):
-    """The operands are the kernels' only 16-byte LDS reads."""
+    """The operands are the kernels' only 16-byte LDS reads: never after a
+    store with nothing between, and two wave barriers for each group of them,
+    one on either side (the later one may stand before the next stores)."""
     assert len(kernels) >= 8
     for name, ops in kernels.items():
-        assert "ds_read_b128" in ops, name
-        last = None  # the last of the accesses below since anything ordered them
+        stored = reading = False  # a store since the last barrier; within a group of reads
+        groups = 0
         for i, op in enumerate(ops):
-            if op in ("wave_barrier", "s_barrier"):
-                last = None
-            elif op == "ds_read_b128" or op.startswith("ds_write"):
-                kind = op[:7]
-                assert last in (None, kind), (name, ops[max(0, i - 12) : i + 1])
-                last = kind
+            if op == "ds_read_b128":
+                assert not stored, (name, ops[max(0, i - 12) : i + 1])
+                groups += not reading
+                reading = True
+            else:
+                reading = False
+                if op in ("wave_barrier", "s_barrier"):
+                    stored = False
+                elif op.startswith("ds_write"):
+                    stored = True
+        assert groups > 0 and ops.count("wave_barrier") >= 2 * groups, (name, groups, ops.count("wave_barrier"))
